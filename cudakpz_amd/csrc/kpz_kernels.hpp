@@ -42,6 +42,25 @@ struct DtPhaseArgs {
 // lanes of a TinyMT32 DT phase with T < nb streams and chains of C blocks
 inline int64_t dt_tmt_lanes(int64_t nb, int64_t T, int C) { return T * (((nb + T - 1) / T + C - 1) / C); }
 hipError_t launch_dt_phase(const DtPhaseArgs& a, hipStream_t stream);
+
+// The same phase with one wave per block (kpz_dt_wave.hip): 16 x 16-site
+// blocks, SLCG64 streams.
+struct DtWaveJumps {
+	Affine lane[6];  // J(draws per update << k): a lane's first update
+	Affine window;   // J(64 draws per update): its next one
+};
+DtWaveJumps dt_wave_jumps(const Affine& step, int drawsPerUpdate);
+// Blocks up to which one wave per block is faster than one lane per block.
+// us per MCS (4 phases), lane / wave: 512^2 (2^8 blocks) KPZ 89 / 22, p/q 117 /
+// 21, disorder 175 / 24; 2048^2 (2^12) 91 / 34, 119 / 32, 177 / 40; 4096^2
+// (2^14) 93 / 91, 121 / 90, 180 / 113.  At 8192^2 (2^16) the wave kernel, bound
+// by instruction issue there, would take four times its 4096^2 figures and the
+// lane kernel 103, 140 and 228.
+constexpr int64_t DT_WAVE_MAX_BLOCKS = 1 << 14;
+// whether the phase takes less time with one wave per block than with one lane
+bool dt_wave_better(int lbx, int lby, int64_t nb, bool tinyMT);
+hipError_t launch_dt_wave(const DtPhaseArgs& a, const DtWaveJumps& J, hipStream_t stream);
+
 // tmtJ for a DT phase with T < nb streams: entry c < n -> x^((c / T) * drawsPerEntry)
 // mod the orbit polynomial of stream c % T (drawsPerEntry: the draws of a chain)
 hipError_t launch_tmt_block_polys(const TmtOrbit* orb, int64_t T, int64_t n, uint64_t drawsPerEntry, Poly128* out,

@@ -521,6 +521,8 @@ void SchedulerDT::run(int n, int upd)
 	a.random_origin = ro_;
 	a.tp = thresh(upd ? p_ : 1.0);
 	a.tq = thresh(upd ? q_ : 0.0);
+	const bool wave = dt_wave_better(lbx_, lby_, nb_, tinyMT());
+	const DtWaveJumps waveJ = wave ? dt_wave_jumps(step_, du) : DtWaveJumps{};
 	for(int m = 0; m < n; ++m)
 	{
 		// SchedulerCPUDT::mcs (kpz/schedulerCPUDT.cpp:65-90) / SchedulerCPUDTr::doMcs
@@ -547,7 +549,7 @@ void SchedulerDT::run(int n, int upd)
 			}
 			a.st_in = stIn();
 			a.st_out = (T_ < nb_) ? stOut() : stIn();
-			check(launch_dt_phase(a, stream_), "dt_phase");
+			check(wave ? launch_dt_wave(a, waveJ, stream_) : launch_dt_phase(a, stream_), "dt_phase");
 			if(T_ < nb_)
 				swapStreams();
 		}
