@@ -801,20 +801,35 @@ SchedulerSCA::SchedulerSCA(int lx, int ly, const Params& p) : SchedulerService(l
 	args_.nV = (int)V.size();
 	for(size_t k = 0; k < V.size(); ++k)
 		args_.V[k] = V[k];
-	args_.rowJ = upload(rowJ, rowJ_);
-	args_.baseJ = upload(baseJ, baseJ_);
-	args_.cellJ = upload(cellJ, cellJ_);
+	std::vector<Affine> tab(rowJ);
+	tab.insert(tab.end(), baseJ.begin(), baseJ.end());
+	tab.insert(tab.end(), cellJ.begin(), cellJ.end());
+	args_.rowJ = upload(tab, jumps_);
+	args_.baseJ = args_.rowJ + rowJ.size();
+	args_.cellJ = args_.baseJ + baseJ.size();
 	args_.fullBig = affine_pow(cell, (uint64_t)nyb * (uint64_t)(pc + 1));
 	args_.fullSmall = affine_pow(cell, (uint64_t)nyb * (uint64_t)pc);
 	args_.step = step_;
-	// band kernel shape: up to 64 cell columns per lane group, 64 cell rows per band
+	// Band kernel shape: up to 64 cell columns per lane group.  A lane walks the
+	// 2^lNB cell rows of its band one after the other, so long bands leave small
+	// lattices with few waves (64 rows: a wave per SIMD at 8192^2); short bands
+	// cost more edge words for the fix kernel.  Bands of 64 rows are halved
+	// while the launch has less than 8192 waves, down to 4 rows, and to 2 rows
+	// below 2048 waves.  us per MCS with 64 rows / so: 512^2 58 / 12.5, 2048^2
+	// 72 / 15.0 (4 rows: 15.8), 4096^2 76 / 20 (2 rows: 24), 8192^2 81 / 40,
+	// 16384^2 120 / 102 (with 4096 waves: 111).
 	args_.lG = std::min(lx - 2, 6);
 	args_.lNB = std::min(ly - 2, 6);
+	const auto waves = [&] { return ((int64_t)dimXW * nyb) >> (6 + args_.lNB); };
+	while(args_.lNB > 2 && waves() < 8192)
+		--args_.lNB;
+	if(args_.lNB == 2 && waves() < 2048)
+		args_.lNB = 1;
 	const size_t groups = (size_t)dimXW >> args_.lG;
-	edgeR_.alloc(std::max<size_t>(1, (size_t)nyb * groups) * 4);
-	edgeU_.alloc(((size_t)nyb >> args_.lNB) * (size_t)dimXW * 4);
-	args_.edgeR = edgeR_.as<uint32_t>();
-	args_.edgeU = edgeU_.as<uint32_t>();
+	const size_t edgeWords = (size_t)nyb * groups;
+	edges_.alloc((edgeWords + ((size_t)nyb >> args_.lNB) * (size_t)dimXW) * 4);
+	args_.edgeR = edges_.as<uint32_t>();
+	args_.edgeU = args_.edgeR + edgeWords;
 }
 
 void SchedulerSCA::mcs(int n)

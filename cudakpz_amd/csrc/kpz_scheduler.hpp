@@ -288,7 +288,7 @@ public:
 private:
 	void run(int n, bool disorder);
 	CbLocalArgs args_{};
-	DevBuf rowJ_, baseJ_, cellJ_, edgeR_, edgeU_;
+	DevBuf jumps_, edges_;
 };
 
 std::unique_ptr<SchedulerService> makeScheduler(int kind, int lx, int ly, const Params& p);
