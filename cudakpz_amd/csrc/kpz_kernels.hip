@@ -2027,24 +2027,67 @@ __device__ __forceinline__ void chunk_prefix2(uint64_t b1, uint64_t b2, int nbit
 	s12 = sab;
 }
 
-__device__ __forceinline__ int64_t wave_incl_scan(int64_t v, int lane)
+// Wave scans and sums on the DPP paths of the VALU: row_shr 1, 2, 4, 8 scan the
+// four rows of 16 lanes, row_bcast15 adds row 0's (2's) total to row 1 (3) and
+// row_bcast31 that of the lower half to the upper one.  A step takes a few
+// cycles, where the same scan with ds_bpermute waits for the LDS in each of its
+// six steps (64-bit sums: 12 round trips).  All lanes of the wave must be here.
+template<int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_from(uint32_t v) // lanes without a source and rows not in ROWS get 0
 {
-#pragma unroll
-	for(int o = 1; o < 64; o <<= 1)
-	{
-		const int64_t u = (int64_t)shfl64((uint64_t)v, lane >= o ? lane - o : lane, 64);
-		if(lane >= o)
-			v += u;
-	}
+	return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+
+template<class F>
+__device__ __forceinline__ void wave_scan_steps(F&& step)
+{
+	step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});
+	step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+	step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+	step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+	step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});
+	step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
+}
+
+__device__ __forceinline__ int wave_incl_scan32(int v)
+{
+	wave_scan_steps([&](auto c, auto r) { v += (int)dpp_from<decltype(c)::value, decltype(r)::value>((uint32_t)v); });
 	return v;
 }
 
-__device__ __forceinline__ int64_t wave_sum(int64_t v)
+__device__ __forceinline__ int64_t wave_incl_scan(int64_t v)
 {
-#pragma unroll
-	for(int o = 32; o > 0; o >>= 1)
-		v += (int64_t)shfl64((uint64_t)v, (threadIdx.x & 63) ^ o, 64);
+	wave_scan_steps([&](auto c, auto r) {
+		const uint32_t lo = dpp_from<decltype(c)::value, decltype(r)::value>((uint32_t)v);
+		const uint32_t hi = dpp_from<decltype(c)::value, decltype(r)::value>((uint32_t)((uint64_t)v >> 32));
+		v += (int64_t)(((uint64_t)hi << 32) | lo);
+	});
 	return v;
+}
+
+// lane 63's value, in every lane
+__device__ __forceinline__ int wave_last32(int v) { return __builtin_amdgcn_readlane(v, 63); }
+__device__ __forceinline__ int64_t wave_last(int64_t v)
+{
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), 63);
+	return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+__device__ __forceinline__ int64_t wave_sum(int64_t v) { return wave_last(wave_incl_scan(v)); }
+
+__device__ __forceinline__ __int128 wave_sum128(__int128 v)
+{
+	wave_scan_steps([&](auto c, auto r) {
+		uint32_t w[4];
+#pragma unroll
+		for(int k = 0; k < 4; ++k)
+			w[k] = dpp_from<decltype(c)::value, decltype(r)::value>((uint32_t)((unsigned __int128)v >> (32 * k)));
+		const uint64_t lo = ((uint64_t)w[1] << 32) | w[0], hi = ((uint64_t)w[3] << 32) | w[2];
+		v += (__int128)(((unsigned __int128)hi << 64) | lo);
+	});
+	const uint64_t lo = (uint64_t)wave_last((int64_t)(uint64_t)v);
+	return ((__int128)wave_last((int64_t)(v >> 64)) << 64) | lo;
 }
 
 // One wave computes the statistics of site row y; lane 0 writes them to o[]
@@ -2084,14 +2127,14 @@ __device__ __forceinline__ void row_stats_row(const uint32_t* __restrict__ lat, 
 				d0s = (bs & 1) ? 1 : -1;
 			}
 		}
-		const int64_t incl = wave_incl_scan(q, lane);
+		const int64_t incl = wave_incl_scan(q);
 		const int64_t c = run + incl - q;
 		S1 += n * c + sq;
 		S2 += n * c * c + 2 * c * sq + sq2;
 		run += (int64_t)shfl64((uint64_t)incl, 63, 64);
 		if(CORR)
 		{
-			const int64_t incs = wave_incl_scan(qs, lane);
+			const int64_t incs = wave_incl_scan(qs);
 			const int64_t cs = runS + incs - qs;
 			T1 += n * cs + ss;
 			T2 += n * cs * cs + 2 * cs * ss + ss2;
@@ -2177,7 +2220,9 @@ __global__ __launch_bounds__(256) void row_stats_local_kernel(const uint32_t* __
 	if(yw >= (1 << (ly - 2)))
 		return; // uniform per wave; no barrier below
 	const int XW = 1 << (lx - 2);
-	const int K = XW < RS_K ? XW : RS_K;     // even: XW >= 2
+	// words per lane and round: as many lanes as there are word pairs, up to
+	// RS_K words each (a row of 128 words: 64 lanes of 2, not 8 of 16)
+	const int K = XW >= 64 * RS_K ? RS_K : (XW > 128 ? XW / 64 : 2);
 	const int span = 64 * K;                 // words per round
 	const uint32_t* __restrict__ row = lat + ((size_t)yw << (lx - 2));
 	int64_t S1[4] = {0, 0, 0, 0}, S2[4] = {0, 0, 0, 0};
@@ -2211,27 +2256,26 @@ __global__ __launch_bounds__(256) void row_stats_local_kernel(const uint32_t* __
 				pair(v.z, v.w);
 			}
 		}
-		else if(live)
+		else if(live && K >= 4)
 		{
-			for(int k = 0; k < K; k += 2)
-				pair(row[wl + k], row[wl + k + 1]);
+			for(int k = 0; k < K; k += 4)
+			{
+				const uint4 v = *reinterpret_cast<const uint4*>(row + wl + k);
+				pair(v.x, v.y);
+				pair(v.z, v.w);
+			}
 		}
+		else if(live)
+			pair(row[wl], row[wl + 1]);
 		const int n = live ? 4 * K : 0;
 #pragma unroll
 		for(int r = 0; r < 4; ++r)
 		{
-			int incl = c[r];
-#pragma unroll
-			for(int o = 1; o < 64; o <<= 1)
-			{
-				const int u = __shfl_up(incl, o, 64);
-				if(lane >= o)
-					incl += u;
-			}
+			const int incl = wave_incl_scan32(c[r]);
 			const int64_t C = (int64_t)base[r] + (incl - c[r]);
 			S1[r] += (int64_t)n * C + s1[r];
 			S2[r] += (int64_t)n * C * C + 2 * C * s1[r] + s2[r];
-			base[r] += __shfl(incl, 63, 64);
+			base[r] += wave_last32(incl);
 		}
 	}
 	const int64_t L = (int64_t)1 << lx;
@@ -2294,7 +2338,7 @@ __global__ __launch_bounds__(256) void row_stats_cbbit_kernel(const uint32_t* __
 	const size_t rowW = (size_t)y << (lx - 6);
 	const uint32_t* __restrict__ ev = lat + rowW + ((y & 1) ? (sw >> 1) : 0);
 	const uint32_t* __restrict__ od = lat + rowW + ((y & 1) ? 0 : (sw >> 1));
-	const int K = WR < CB_RS_K ? WR : CB_RS_K;
+	const int K = WR >= 64 * CB_RS_K ? CB_RS_K : (WR > 64 ? WR / 64 : 1);
 	const int span = 64 * K;
 	int64_t S1 = 0, S2 = 0;
 	int base = 0;
@@ -2335,18 +2379,11 @@ __global__ __launch_bounds__(256) void row_stats_cbbit_kernel(const uint32_t* __
 				pair(ev[wl + k], od[wl + k]);
 		}
 		const int n = live ? 64 * K : 0;
-		int incl = c;
-#pragma unroll
-		for(int o = 1; o < 64; o <<= 1)
-		{
-			const int u = __shfl_up(incl, o, 64);
-			if(lane >= o)
-				incl += u;
-		}
+		const int incl = wave_incl_scan32(c);
 		const int64_t C = (int64_t)base + (incl - c);
 		S1 += (int64_t)n * C + s1;
 		S2 += (int64_t)n * C * C + 2 * C * s1 + s2;
-		base += __shfl(incl, 63, 64);
+		base += wave_last32(incl);
 	}
 	const int64_t L = (int64_t)1 << lx;
 	const int64_t sp = wave_sum(S1), spp = wave_sum(S2);
@@ -2715,23 +2752,6 @@ __global__ __launch_bounds__(256) void row_stats_kernel(const uint32_t* __restri
 constexpr int RC_ROWS = 256;
 enum { RC_DA, RC_DB, RC_A1, RC_A2LO, RC_A2HI, RC_T1, RC_B12LO, RC_B12HI, RC_TCS, RC_N, RC_H, RC_G, RC_REC };
 
-__device__ __forceinline__ __int128 wave_sum128(__int128 v)
-{
-	uint64_t lo = (uint64_t)v;
-	int64_t hi = (int64_t)(v >> 64);
-#pragma unroll
-	for(int o = 32; o > 0; o >>= 1)
-	{
-		const int src = (threadIdx.x & 63) ^ o;
-		const uint64_t lo2 = shfl64(lo, src, 64);
-		const int64_t hi2 = (int64_t)shfl64((uint64_t)hi, src, 64);
-		const uint64_t s = lo + lo2;
-		hi = hi + hi2 + (s < lo ? 1 : 0);
-		lo = s;
-	}
-	return ((__int128)hi << 64) | lo;
-}
-
 __global__ __launch_bounds__(RC_ROWS) void row_part_kernel(const int64_t* __restrict__ rows, int lx, int ly, int corr,
 		int64_t* __restrict__ hsRel, int64_t* __restrict__ part)
 {
@@ -2762,7 +2782,7 @@ __global__ __launch_bounds__(RC_ROWS) void row_part_kernel(const int64_t* __rest
 	const int64_t sy = o3 ? 1 : -1, syS = o6 ? 1 : -1;
 	const int64_t da = live ? sy + o2 : 0, db = (live && corr) ? syS + o5 : 0;
 	// workgroup exclusive scan of the row changes
-	const int64_t ia = wave_incl_scan(da, lane), ib = corr ? wave_incl_scan(db, lane) : 0;
+	const int64_t ia = wave_incl_scan(da), ib = corr ? wave_incl_scan(db) : 0;
 	if(lane == 63)
 	{
 		wa[wv] = ia;
@@ -2844,14 +2864,60 @@ __global__ __launch_bounds__(RC_ROWS) void row_part_kernel(const int64_t* __rest
 	}
 }
 
+// Sums of a workgroup of up to 16 waves, written to res by its first wave
+struct WgTotals {
+	int64_t s1, t1, tcs;
+	__int128 s2, s12;
+};
+__device__ __forceinline__ void workgroup_totals(const WgTotals& v, int corr, int64_t* __restrict__ res)
+{
+	__shared__ int64_t q1[16], qt[16], qc[16];
+	__shared__ __int128 q2[16], q12[16];
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+	const int64_t s1 = wave_sum(v.s1);
+	const __int128 s2 = wave_sum128(v.s2);
+	int64_t t1 = 0, tcs = 0;
+	__int128 s12 = 0;
+	if(corr)
+	{
+		t1 = wave_sum(v.t1);
+		s12 = wave_sum128(v.s12);
+		tcs = wave_sum(v.tcs);
+	}
+	if(lane == 0)
+	{
+		q1[wv] = s1;
+		q2[wv] = s2;
+		qt[wv] = t1;
+		q12[wv] = s12;
+		qc[wv] = tcs;
+	}
+	__syncthreads();
+	if(wv)
+		return;
+	const bool has = lane < nw;
+	const int64_t S1 = wave_sum(has ? q1[lane & 15] : 0);
+	const __int128 S2 = wave_sum128(has ? q2[lane & 15] : 0);
+	const int64_t T1 = wave_sum(has ? qt[lane & 15] : 0), TC = wave_sum(has ? qc[lane & 15] : 0);
+	const __int128 S12 = wave_sum128(has ? q12[lane & 15] : 0);
+	if(lane == 0)
+	{
+		res[0] = S1;
+		res[1] = (int64_t)(uint64_t)S2;
+		res[2] = (int64_t)(S2 >> 64);
+		res[3] = corr ? T1 : 0;
+		res[4] = corr ? (int64_t)(uint64_t)S12 : 0;
+		res[5] = corr ? (int64_t)(S12 >> 64) : 0;
+		res[6] = corr ? TC : 0;
+	}
+}
+
 // pass 2: one 1024-lane workgroup over the nb records; lane i takes records
 // [i R, (i+1) R); writes every record's start heights H, G (for pass 3)
 __global__ __launch_bounds__(1024) void row_final_kernel(int64_t* __restrict__ part, int64_t nb, int lx, int corr,
 		int64_t* __restrict__ res)
 {
 	__shared__ int64_t sa[16], sb[16];
-	__shared__ int64_t q1[16], qt[16], qc[16];
-	__shared__ __int128 q2[16], q12[16];
 	const int i = threadIdx.x, lane = i & 63, wv = i >> 6;
 	const int64_t R = (nb + 1023) / 1024;
 	const int64_t b0 = i * R, b1 = (b0 + R < nb) ? b0 + R : nb;
@@ -2861,7 +2927,7 @@ __global__ __launch_bounds__(1024) void row_final_kernel(int64_t* __restrict__ p
 		da += part[b * RC_REC + RC_DA];
 		db += part[b * RC_REC + RC_DB];
 	}
-	const int64_t ia = wave_incl_scan(da, lane), ib = wave_incl_scan(db, lane);
+	const int64_t ia = wave_incl_scan(da), ib = wave_incl_scan(db);
 	if(lane == 63)
 	{
 		sa[wv] = ia;
@@ -2897,40 +2963,69 @@ __global__ __launch_bounds__(1024) void row_final_kernel(int64_t* __restrict__ p
 		H += r[RC_DA];
 		G += r[RC_DB];
 	}
-	s1 = wave_sum(s1);
-	s2 = wave_sum128(s2);
-	t1 = wave_sum(t1);
-	s12 = wave_sum128(s12);
-	tcs = wave_sum(tcs);
-	if(lane == 0)
+	workgroup_totals({s1, t1, tcs, s2, s12}, corr, res);
+}
+
+// Both passes at once for up to RT_ROWS rows: one workgroup, a row per lane.
+// On such lattices the two passes and the gap between them took longer than
+// the rows' own statistics.  A whole w^2 sample in us, two passes / one: 512
+// rows 38 / 20 (with the DPP sums and the totals written to host memory), 2048
+// rows with two rows per lane 22.6 / 24.5, 4096 with four 22.9 / 30.5.  hs
+// receives every row's start height.
+constexpr int64_t RT_ROWS = 1024;
+
+__global__ __launch_bounds__(1024) void row_total_kernel(const int64_t* __restrict__ rows, int lx, int ly, int corr,
+		int64_t* __restrict__ hs, int64_t* __restrict__ res)
+{
+	__shared__ int64_t sa[16], sb[16];
+	const int i = threadIdx.x, lane = i & 63, wv = i >> 6, nw = (int)blockDim.x >> 6;
+	const int ny = 1 << ly;
+	int64_t o[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, da = 0, db = 0;
+	if(i < ny)
 	{
-		q1[wv] = s1;
-		q2[wv] = s2;
-		qt[wv] = t1;
-		q12[wv] = s12;
-		qc[wv] = tcs;
+		const int64_t* row = rows + (size_t)i * ROW_STATS;
+#pragma unroll
+		for(int k = 0; k < 9; ++k)
+			if(k < 4 || corr)
+				o[k] = row[k];
+		da = (o[3] ? 1 : -1) + o[2];
+		if(corr)
+			db = (o[6] ? 1 : -1) + o[5];
+	}
+	const int64_t ia = wave_incl_scan(da), ib = corr ? wave_incl_scan(db) : 0;
+	if(lane == 63)
+	{
+		sa[wv] = ia;
+		sb[wv] = ib;
 	}
 	__syncthreads();
-	if(i == 0)
-	{
-		int64_t S1 = 0, T1 = 0, TC = 0;
-		__int128 S2 = 0, S12 = 0;
-		for(int k = 0; k < 16; ++k)
+	int64_t H = ia - da, G = ib - db;
+#pragma unroll
+	for(int k = 0; k < 16; ++k)
+		if(k < nw)
 		{
-			S1 += q1[k];
-			S2 += q2[k];
-			T1 += qt[k];
-			S12 += q12[k];
-			TC += qc[k];
+			const int64_t a = sa[k], b = sb[k];
+			H += k < wv ? a : 0;
+			G += k < wv ? b : 0;
 		}
-		res[0] = S1;
-		res[1] = (int64_t)(uint64_t)S2;
-		res[2] = (int64_t)(S2 >> 64);
-		res[3] = corr ? T1 : 0;
-		res[4] = corr ? (int64_t)(uint64_t)S12 : 0;
-		res[5] = corr ? (int64_t)(S12 >> 64) : 0;
-		res[6] = corr ? TC : 0;
+	const int64_t L = (int64_t)1 << lx;
+	WgTotals v{0, 0, 0, 0, 0};
+	if(i < ny)
+	{
+		H += o[3] ? 1 : -1; // the row's start height
+		if(hs)
+			hs[i] = H;
+		v.s1 = L * H + o[0];
+		v.s2 = (__int128)L * H * H + (__int128)2 * H * o[0] + o[1];
+		if(corr)
+		{
+			G += o[6] ? 1 : -1;
+			v.t1 = L * G + o[4];
+			v.s12 = (__int128)L * H * G + (__int128)H * o[4] + (__int128)G * o[0] + o[7];
+			v.tcs = o[8];
+		}
 	}
+	workgroup_totals(v, corr, res);
 }
 
 // pass 3 (hs requested): every row's start height = its workgroup's H plus
@@ -2977,7 +3072,7 @@ __global__ __launch_bounds__(256) void row_moments_kernel(const uint32_t* __rest
 			if(j == 0)
 				d0 = (b & 1) ? 1 : -1;
 		}
-		const int64_t incl = wave_incl_scan(q, lane);
+		const int64_t incl = wave_incl_scan(q);
 		int64_t h = h0 + run + incl - q;
 		if(valid)
 		{
@@ -3393,7 +3488,7 @@ __global__ __launch_bounds__(BC_WG) void batch_combine_kernel(const BatchRep* __
 		rel = hs + s[2];
 	}
 	const int64_t n = y1 - y0;
-	const int64_t inc = wave_incl_scan(rel, lane);
+	const int64_t inc = wave_incl_scan(rel);
 	if(lane == 63)
 		wd[wv] = inc;
 	__syncthreads();
@@ -3734,13 +3829,20 @@ unsigned corr_grid(int64_t units)
 }
 } // namespace
 
+// log2 of the sites from which the correlator takes the table kernel: building
+// its 129 KiB of tables takes 25 us, which the per-site kernel does not need.
+// A whole correlator sample in us, per site / tables: ENC_LOCAL 512^2 31 / 53,
+// 2048^2 35 / 56, 4096^2 (2^24) 42 / 56, 8192^2 90 / 66; ENC_CBBIT 28 / 53, 32 /
+// 51, 34 / 50, 64 / 61.
+constexpr int CORR_TABLE_MIN_LOG2 = 25;
+
 hipError_t launch_row_stats(const uint32_t* lat, const uint32_t* snap, int enc, int lx, int ly,
 		int64_t* out, hipStream_t stream)
 {
 	const dim3 grid((unsigned)(((1 << ly) + 3) / 4));
 	if(enc == ENC_LOCAL)
 	{
-		if(snap && lx >= 3 && ly >= 2)
+		if(snap && lx >= 3 && ly >= 2 && lx + ly >= CORR_TABLE_MIN_LOG2)
 			hipLaunchKernelGGL(row_corr_table_kernel<ENC_LOCAL>, dim3(corr_grid(1ll << (ly - 2))), dim3(CORR_WG), 0,
 			                   stream, lat, snap, lx, ly, out);
 		else if(snap)
@@ -3754,7 +3856,7 @@ hipError_t launch_row_stats(const uint32_t* lat, const uint32_t* snap, int enc, 
 	}
 	else
 	{
-		if(snap && lx >= 6)
+		if(snap && lx >= 6 && lx + ly >= CORR_TABLE_MIN_LOG2)
 			hipLaunchKernelGGL(row_corr_table_kernel<ENC_CBBIT>, dim3(corr_grid(1ll << ly)), dim3(CORR_WG), 0,
 			                   stream,
 			                   lat, snap, lx, ly, out);
@@ -3779,6 +3881,12 @@ hipError_t launch_row_combine(const int64_t* rows, int lx, int ly, bool corr, in
 {
 	if(!rows || !part || !res || lx < 0 || ly < 0 || lx > 30 || ly > 30)
 		return hipErrorInvalidValue;
+	if(((int64_t)1 << ly) <= RT_ROWS)
+	{
+		const int lanes = (1 << ly) < 64 ? 64 : 1 << ly;
+		hipLaunchKernelGGL(row_total_kernel, dim3(1), dim3(lanes), 0, stream, rows, lx, ly, corr ? 1 : 0, hs, res);
+		return hipGetLastError();
+	}
 	const int64_t nb = (((int64_t)1 << ly) + RC_ROWS - 1) / RC_ROWS;
 	hipLaunchKernelGGL(row_part_kernel, dim3((unsigned)nb), dim3(RC_ROWS), 0, stream, rows, lx, ly, corr ? 1 : 0, hs,
 	                   part);

@@ -37,6 +37,27 @@ void DevBuf::alloc(size_t bytes)
 	n_ = bytes;
 }
 
+PinnedBuf::~PinnedBuf()
+{
+	if(p_)
+		(void)hipHostFree(p_);
+}
+
+void PinnedBuf::alloc(size_t bytes)
+{
+	if(p_)
+	{
+		(void)hipHostFree(p_);
+		p_ = nullptr;
+	}
+	const hipError_t e = hipHostMalloc(&p_, bytes, hipHostMallocDefault);
+	if(e != hipSuccess)
+	{
+		p_ = nullptr;
+		throw Error(-3, "hipHostMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
+	}
+}
+
 // ======================================================================
 SchedulerService::SchedulerService(int lx, int ly, Encoding enc, const Params& p)
 	: params_(p), size_{lx, ly}, enc_(enc), T_(p.threads), S_(p.skip), device_(p.device)
@@ -318,9 +339,8 @@ Sums SchedulerService::totals(const uint32_t* snap, int64_t* hs)
 	check(launch_row_combine(rows_.as<int64_t>(), size_.lx, size_.ly, snap != nullptr, hs,
 	                         rows_.as<int64_t>() + (size_t)size_.dimY() * ROW_STATS, totals_.as<int64_t>(), stream_),
 	      "row_combine");
-	int64_t r[7];
-	check(hipMemcpyAsync(r, totals_.get(), sizeof r, hipMemcpyDeviceToHost, stream_), "totals D2H");
 	sync();
+	const volatile int64_t* const r = totals_.as<int64_t>(); // host memory, written by the kernel
 	Sums s;
 	s.sumH = r[0];
 	s.sumH2 = ((__int128)r[2] << 64) | (uint64_t)r[1];

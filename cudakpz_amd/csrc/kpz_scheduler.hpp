@@ -48,6 +48,20 @@ private:
 	size_t n_ = 0;
 };
 
+// page-locked host memory that kernels write results to directly
+class PinnedBuf {
+public:
+	PinnedBuf() = default;
+	~PinnedBuf();
+	PinnedBuf(const PinnedBuf&) = delete;
+	PinnedBuf& operator=(const PinnedBuf&) = delete;
+	void alloc(size_t bytes);
+	template<class T> T* as() const { return (T*)p_; }
+
+private:
+	void* p_ = nullptr;
+};
+
 void check(hipError_t e, const char* what);
 
 struct Params {
@@ -200,7 +214,8 @@ protected:
 	};
 	Sums correlateWith(const DevBuf& snap);
 	Sums totals(const uint32_t* snap, int64_t* hs);
-	DevBuf lat_, rows_, totals_, rowStart_, rowMoments_, check_;
+	DevBuf lat_, rows_, rowStart_, rowMoments_, check_;
+	PinnedBuf totals_;
 	void consistencyOf(const uint32_t* lat, int64_t out[3]);
 	std::vector<Tag> tags_;
 	DevBuf st_[2];
