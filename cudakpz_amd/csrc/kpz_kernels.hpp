@@ -97,6 +97,25 @@ struct CbHalfArgs {
 	const void* rnd;
 };
 hipError_t launch_cbbit_half(const CbHalfArgs& a, hipStream_t stream);
+
+// ---- SCABit: both bit-parallel half-sweeps (mode 0) of an MCS in one pass ----
+// (kpz_cbbit_mcs.hip), from one lattice into another; lx >= 7
+constexpr int CBBIT_MCS_MAX_LX = 18; // a row is a workgroup of 1024 lanes then
+int cbbit_mcs_band(int lx, int ly);  // log2 rows of a band
+struct CbMcsArgs {
+	const uint32_t* src;
+	uint32_t* dst;
+	int lx, ly;
+	const uint64_t* st_in;
+	uint64_t* st_out;       // != st_in; the streams after both half-sweeps
+	int T, per, rem;        // as CbHalfArgs
+	const Affine* rowJ;
+	const Affine* wordJ;    // wordJ[w]: skip w words of draws, all words of a row
+	Affine step, fullBig, fullSmall;
+	int lR;                 // log2 rows of a band
+};
+hipError_t launch_cbbit_mcs(const CbMcsArgs& a, hipStream_t stream);
+
 // TinyMT32 workers of SCABit: the random part of one half-sweep (mode 0 VL3,
 // 1 per-site pq, 2 disorder) into `out`, one lane per 1/2^lC of a row;
 // streams read from gin, the state after the half-sweep written to gout (7

@@ -418,7 +418,17 @@ void SchedulerService::moments(long double out[7])
 void SchedulerService::correlateTag(unsigned int stop)
 {
 	Tag t;
-	t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
+	try
+	{
+		t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
+	}
+	catch(const Error&)
+	{
+		if(!dropSpare())
+			throw;
+		(void)hipGetLastError();
+		t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
+	}
 	t.mcs = mcs_;
 	t.stop = stop;
 	const uint64_t bytes = size_.sizeW() * 4;
@@ -643,6 +653,53 @@ SchedulerSCABit::Tables& SchedulerSCABit::tables(int mode)
 	return ref;
 }
 
+// Whether bit-parallel MCS run in one pass (kpz_cbbit_mcs.hip), for which the
+// scheduler keeps a second lattice.  It is taken only for lattices of at most
+// 4 GiB and only while three quarters of the device's memory stay free, so that
+// programs that fill the memory with lattices or tags find it as before.
+bool SchedulerSCABit::wholeMcs()
+{
+	if(wholeMcs_ != UNKNOWN)
+		return wholeMcs_ == YES;
+	wholeMcs_ = NO;
+	const size_t bytes = (size_t)size_.sizeW() * 4;
+	if(size_.lx < 7 || size_.lx > CBBIT_MCS_MAX_LX || bytes > ((size_t)4 << 30))
+		return false;
+	size_t free = 0, total = 0;
+	if(hipMemGetInfo(&free, &total) != hipSuccess || free < bytes || free - bytes < total / 4 * 3)
+		return false;
+	try
+	{
+		alt_.alloc(bytes);
+	}
+	catch(const Error&)
+	{
+		(void)hipGetLastError();
+		return false;
+	}
+	std::vector<Affine> word((size_t)1 << (size_.lx - 7));
+	const Affine wordStep = affine_pow(step_, 2);
+	Affine acc{1, 0};
+	for(auto& j : word)
+	{
+		j = acc;
+		acc = compose(wordStep, acc);
+	}
+	upload(word, wordJ_);
+	wholeMcs_ = YES;
+	return true;
+}
+
+bool SchedulerSCABit::dropSpare()
+{
+	if(!alt_.get())
+		return false;
+	sync();
+	alt_.alloc(0);
+	wholeMcs_ = NO;
+	return true;
+}
+
 void SchedulerSCABit::run(int n, int mode)
 {
 	if(mode == 2 && !hasDisorder())
@@ -729,6 +786,34 @@ void SchedulerSCABit::run(int n, int mode)
 	a.tp = thresh23(p_);
 	a.tq = thresh23(q_);
 	a.lG = lG_;
+	// (asked for on any first call: later ones may be under capture)
+	if(mode == 0 && wholeMcs())
+	{
+		// pairs of whole MCS, so that the lattice stays where it is
+		CbMcsArgs w{};
+		w.lx = size_.lx;
+		w.ly = size_.ly;
+		w.T = (int)T_;
+		w.per = per_;
+		w.rem = rem_;
+		w.rowJ = a.rowJ;
+		w.wordJ = wordJ_.as<Affine>();
+		w.step = step_;
+		w.fullBig = a.fullBig;
+		w.fullSmall = a.fullSmall;
+		w.lR = cbbit_mcs_band(size_.lx, size_.ly);
+		for(; n >= 2; n -= 2)
+			for(int k = 0; k < 2; ++k)
+			{
+				w.src = k ? alt_.as<uint32_t>() : deviceLattice();
+				w.dst = k ? deviceLattice() : alt_.as<uint32_t>();
+				w.st_in = stIn();
+				w.st_out = stOut();
+				check(launch_cbbit_mcs(w, stream_), "cbbit_mcs");
+				swapStreams();
+				++mcs_;
+			}
+	}
 	for(int m = 0; m < n; ++m)
 	{
 		// SchedulerCPUCBBit::doMcs (kpz/schedulerCPUCBBit.cpp:64-78)

@@ -212,6 +212,8 @@ protected:
 		std::unique_ptr<DevBuf> snap;
 		unsigned int mcs, stop;
 	};
+	// gives back memory that only makes calls faster; false if there is none
+	virtual bool dropSpare() { return false; }
 	Sums correlateWith(const DevBuf& snap);
 	Sums totals(const uint32_t* snap, int64_t* hs);
 	DevBuf lat_, rows_, rowStart_, rowMoments_, check_;
@@ -286,8 +288,14 @@ private:
 	};
 	void run(int n, int mode);
 	Tables& tables(int mode);
+	bool wholeMcs();
+	bool dropSpare() override;
 	int per_, rem_, lG_;
 	std::map<int, std::unique_ptr<Tables>> tab_;
+	// bit-parallel MCS in one pass: the other lattice and the jumps to every word
+	// of a row; wholeMcs_: not asked for yet, in use, not to be had
+	DevBuf alt_, wordJ_;
+	enum { UNKNOWN, YES, NO } wholeMcs_ = UNKNOWN;
 };
 
 // Checkerboard SCA on ENC_LOCAL: SchedulerCPUCB semantics (the CPU
