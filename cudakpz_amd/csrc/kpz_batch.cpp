@@ -29,6 +29,18 @@ Batch::Batch(const std::vector<ReplicaSpec>& specs, const BatchTuning& tune, int
 	for(auto& e : copied_)
 		check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
 
+	const bool bySize = tune_.maxLanesLog2 == BatchTuning::LANES_BY_SIZE;
+	if(bySize)
+		tune_.maxLanesLog2 = batch_row_split([&](int l) {
+			int64_t n = 0;
+			for(const ReplicaSpec& s : specs)
+				if(s.kind == KIND_SCABIT)
+				{
+					const bool wide = s.lx >= 7 && ((s.p == 0.5 && s.q == 0.0) || tune_.pqWords64);
+					n += 1ll << (std::max(0, std::min(24, s.ly)) + std::max(0, std::min(s.lx - (wide ? 7 : 6), l)));
+				}
+			return n;
+		});
 	reps_.resize(specs.size());
 	uint64_t latBytes = 0, stWords = 0, tabEntries = 1; // entry 0: identity
 	for(size_t r = 0; r < specs.size(); ++r)
@@ -63,7 +75,7 @@ Batch::Batch(const std::vector<ReplicaSpec>& specs, const BatchTuning& tune, int
 			d.wide = (s.lx >= 7 && (d.mode == 0 || tune_.pqWords64)) ? 1 : 0;
 			const int lWn = s.lx - (d.wide ? 7 : 6);
 			d.lG = std::min(lWn, std::max(0, std::min(6, tune_.maxLanesLog2)));
-			if(s.ly + d.lG < 6)
+			if(s.ly + (bySize ? std::min(lWn, 3) : d.lG) < 6)
 				throw Error(-1, "batch SCABit replica too small for one wave (rows x lanes < 64)");
 			R.T = 1ll << s.ly;
 			d.tp = thresh23(s.p);
@@ -350,6 +362,7 @@ Batch::Chunk& Batch::graphFor(int b, int len)
 		da.nlanes = dtLanes_[g];
 		da.nstatic = dtStatic_[g];
 	}
+	const bool wave = dtLanes_[0] + dtLanes_[1] <= DT_WAVE_MAX_BLOCKS;
 	BatchCbArgs cg[2];
 	for(int g = 0; g < 2; ++g)
 	{
@@ -367,7 +380,7 @@ Batch::Chunk& Batch::graphFor(int b, int len)
 					dg[g].m = m;
 					dg[g].d = d;
 					if(dg[g].nlanes > 0)
-						check(launch_batch_dt(dg[g], dtStream[g]), "batch_dt");
+						check(wave ? launch_batch_dt_wave(dg[g], dtStream[g]) : launch_batch_dt(dg[g], dtStream[g]), "batch_dt");
 				}
 		if(hasCb_)
 			for(int g = 0; g < 2; ++g)

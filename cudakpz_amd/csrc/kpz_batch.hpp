@@ -31,6 +31,7 @@ struct ReplicaSpec {
 
 // performance knobs; none of them changes any replica's result
 struct BatchTuning {
+	static constexpr int LANES_BY_SIZE = -1000; // maxLanesLog2 chosen for the batch (batch_row_split)
 	int maxLanesLog2 = 3;  // SCABit: lanes per row = min(words per row, 2^this)
 	int pqWords64 = 1;     // SCABit per-site replicas: 64-bit (1) or 32-bit (0) words
 	int chunk = 50;        // MCS per captured graph

@@ -577,10 +577,13 @@ int kpz_batch_create(const kpz_replica* reps, int n, const kpz_batch_tuning* tun
 	if(!to_specs(reps, n, specs))
 		return fail(KPZ_EINVAL, "no replicas");
 	return guard([&] {
+		kpz::BatchTuning t = to_tuning(tuning);
+		if(!tuning)
+			t.maxLanesLog2 = kpz::BatchTuning::LANES_BY_SIZE;
 		auto h = new kpz_batch;
 		try
 		{
-			h->b = std::make_unique<kpz::Batch>(specs, to_tuning(tuning), device);
+			h->b = std::make_unique<kpz::Batch>(specs, t, device);
 		}
 		catch(...)
 		{

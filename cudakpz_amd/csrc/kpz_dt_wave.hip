@@ -75,16 +75,12 @@ __device__ __forceinline__ uint32_t from_prev(uint32_t v)
 
 // UPD: 0 = KPZ (pqOneUpdate), 1 = pqSyncRngUpdate, 2 = disorder2SyncRngUpdate,
 // 3 = EW; RO: random origin (as dt_phase_kernel)
+// block i of nb, with this wave's LDS `masks`
 template<int UPD, bool RO>
-__global__ __launch_bounds__(64 * DW_WAVES) void dt_wave_kernel(DtPhaseArgs a, DtWaveJumps J, int64_t nb)
+__device__ __forceinline__ void dt_wave_block(const DtPhaseArgs& a, const DtWaveJumps& J, int64_t i, int64_t nb,
+                                              uint64_t* masks)
 {
-	__shared__ __align__(16) uint64_t shared[DW_WAVES][4 * DW_SITES];
 	const int lane = threadIdx.x & 63;
-	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-	const int64_t i = (int64_t)blockIdx.x * DW_WAVES + wave;
-	if(i >= nb)
-		return; // whole wave; no barrier in this kernel
-	uint64_t* const masks = shared[wave];
 
 	// ---- the block's stream (dt_phase_kernel: DtSlcg::begin)
 	const bool ownStream = a.T >= nb;
@@ -305,6 +301,65 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dt_wave_kernel(DtPhaseArgs a, D
 		a.st_out[t] = a.blockJ(s0);
 }
 
+template<int UPD, bool RO>
+__global__ __launch_bounds__(64 * DW_WAVES) void dt_wave_kernel(DtPhaseArgs a, DtWaveJumps J, int64_t nb)
+{
+	__shared__ __align__(16) uint64_t masks[DW_WAVES][4 * DW_SITES];
+	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+	const int64_t i = (int64_t)blockIdx.x * DW_WAVES + wave;
+	if(i >= nb)
+		return; // whole wave; no barrier in this kernel
+	dt_wave_block<UPD, RO>(a, J, i, nb, masks[wave]);
+}
+
+// One DT phase of every DT (DTr: RO) replica of a batch: entry of the lane
+// table -> wave (batch_dt_kernel takes a lane for each)
+template<bool RO>
+__global__ __launch_bounds__(64 * DW_WAVES) void batch_dt_wave_kernel(BatchDtArgs a)
+{
+	__shared__ __align__(16) uint64_t masks[DW_WAVES][4 * DW_SITES];
+	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+	const int64_t e = (int64_t)blockIdx.x * DW_WAVES + wave + (RO ? a.nstatic : 0);
+	if(e >= (RO ? a.nlanes : a.nstatic))
+		return; // whole wave, here and below
+	const uint2 w = a.lanes[e];
+	if(w.x == 0xFFFFFFFFu || (a.limit && a.m >= a.limit[w.x]))
+		return;
+	const BatchRep& rep = a.reps[w.x];
+	DtPhaseArgs p{};
+	p.lat = rep.lat;
+	p.lx = rep.lx;
+	p.ly = rep.ly;
+	p.st_in = p.st_out = rep.st[0];
+	p.step = rep.step;
+	p.blockJ = rep.full;
+	p.tp = rep.tp;
+	p.tq = rep.tq;
+	const size_t mi = (size_t)a.m * a.nreps + w.x;
+	p.ds = (a.order[mi] >> (2 * a.d)) & 3;
+	if constexpr(RO)
+	{
+		const uint16_t sh = a.shift[mi];
+		p.sx = sh & 0xFF;
+		p.sy = sh >> 8;
+	}
+	const int64_t nb = 1ll << (rep.lx + rep.ly - 10);
+	p.T = nb;
+	// dt_wave_jumps on the scalar unit
+	DtWaveJumps J;
+	J.lane[0] = compose(rep.step, rep.step);
+	if(rep.mode)
+		J.lane[0] = compose(rep.step, J.lane[0]);
+#pragma unroll
+	for(int k = 1; k < 6; ++k)
+		J.lane[k] = compose(J.lane[k - 1], J.lane[k - 1]);
+	J.window = compose(J.lane[5], J.lane[5]);
+	if(rep.mode)
+		dt_wave_block<1, RO>(p, J, w.y, nb, masks[wave]);
+	else
+		dt_wave_block<0, RO>(p, J, w.y, nb, masks[wave]);
+}
+
 template<int UPD>
 void launch(const DtPhaseArgs& a, const DtWaveJumps& J, int64_t nb, hipStream_t stream)
 {
@@ -350,6 +405,18 @@ hipError_t launch_dt_wave(const DtPhaseArgs& a, const DtWaveJumps& J, hipStream_
 		case 3: launch<3>(a, J, nb, stream); break;
 		default: return hipErrorInvalidValue;
 	}
+	return hipGetLastError();
+}
+
+hipError_t launch_batch_dt_wave(const BatchDtArgs& a, hipStream_t stream)
+{
+	if(a.nstatic < 0 || a.nstatic > a.nlanes)
+		return hipErrorInvalidValue;
+	auto grid = [](int64_t n) { return dim3((unsigned)((n + DW_WAVES - 1) / DW_WAVES)); };
+	if(a.nstatic > 0)
+		hipLaunchKernelGGL(batch_dt_wave_kernel<false>, grid(a.nstatic), dim3(64 * DW_WAVES), 0, stream, a);
+	if(a.nlanes > a.nstatic)
+		hipLaunchKernelGGL(batch_dt_wave_kernel<true>, grid(a.nlanes - a.nstatic), dim3(64 * DW_WAVES), 0, stream, a);
 	return hipGetLastError();
 }
 

@@ -244,6 +244,11 @@ struct BatchDtArgs {
 	const int* limit;       // optional [r]: replica r only runs MCS m < limit[r]
 };
 hipError_t launch_batch_dt(const BatchDtArgs& a, hipStream_t stream);
+// the same with one wave per block; better while all blocks that run at the
+// same time are at most DT_WAVE_MAX_BLOCKS (12 DTr jobs of L = 2^8..2^11: 67 ms
+// with a lane per block, 40 so; 107 replicas of L = 2^6..2^10, 7 MCS and w^2:
+// 1.27 and 0.83 ms)
+hipError_t launch_batch_dt_wave(const BatchDtArgs& a, hipStream_t stream);
 
 struct BatchCbArgs {
 	const BatchRep* reps;
@@ -255,6 +260,21 @@ struct BatchCbArgs {
 	const int* limit;       // optional [r]: replica r only runs MCS m < limit[r]
 };
 hipError_t launch_batch_cbbit(const BatchCbArgs& a, hipStream_t stream);
+// log2 lanes that share a SCABit row of a batch or tick: `lanes(l)` is the
+// number of lanes with at most 2^l per row
+template<class F>
+int batch_row_split(F&& lanes)
+{
+	// 8 lanes per row spread a lane's stream set-up (dependent loads of the job
+	// table, the stream and its jumps) over most words; more of them where that
+	// would leave fewer than 4096 waves, as for the last jobs of a server.  32
+	// jobs of L = 2^8..2^13, 100..1000 MCS: 39.4 ms with 8 lanes throughout, 35.5
+	// so, 36.4 with a target of 8192 waves; 1024 replicas are the same with each
+	int l = 3;
+	while(l < 6 && lanes(l) < ((int64_t)4096 << 6))
+		++l;
+	return l;
+}
 
 // lanes per site row in the batched row statistics: one per 64-site chunk, at
 // most 64; a wave takes 64 / batch_row_lanes(lx) consecutive rows of a replica

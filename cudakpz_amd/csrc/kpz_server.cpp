@@ -7,9 +7,6 @@
 namespace kpz {
 
 namespace {
-// log2 of the most lanes that share one SCABit row of a job
-constexpr int SERVE_MAX_LANES_LOG2 = 3;
-
 int ceilLog2(size_t v)
 {
 	int l = 0;
@@ -274,11 +271,6 @@ bool Server::admit(Job& j, PinnedStage& stage)
 		d.kind = BK_SCABIT;
 		d.mode = (s.p == 0.5 && s.q == 0.0) ? 0 : 1;
 		d.wide = s.lx >= 7 ? 1 : 0;
-		// at most 8 lanes per row: a lane then walks >= 8 words of a wide row,
-		// so its stream set-up (dependent loads of the job table, the stream
-		// and its jumps) is spread over >= 512 sites (the choice the batch
-		// autotuner makes on the 4096-replica mix)
-		d.lG = std::min(s.lx - (d.wide ? 7 : 6), SERVE_MAX_LANES_LOG2);
 		j.T = 1ll << s.ly;
 	}
 	else
@@ -310,7 +302,8 @@ bool Server::admit(Job& j, PinnedStage& stage)
 	{
 		const uint64_t du = d.mode == 0 ? (d.wide ? 2 : 1) : (d.wide ? 64 : 32);
 		const uint64_t Wn = 1ull << (s.lx - (d.wide ? 7 : 6));
-		const int G = 1 << d.lG;
+		// jumps for the most lanes per row; rebuild() chooses how many share a row
+		const int G = (int)std::min<uint64_t>(Wn, 64);
 		Affine* lane = (Affine*)stage.take((size_t)G * sizeof(Affine));
 		const Affine word = affine_pow(d.step, du);
 		Affine acc{1, 0};
@@ -321,7 +314,6 @@ bool Server::admit(Job& j, PinnedStage& stage)
 		}
 		d.laneJ = (const Affine*)(base + j.off[2]);
 		check(hipMemcpyAsync((void*)d.laneJ, lane, (size_t)G * sizeof(Affine), hipMemcpyHostToDevice, s0_), "lane table");
-		d.stepJ = affine_pow(d.step, du * (uint64_t)G);
 		d.full = affine_pow(d.step, du * Wn);
 	}
 	else
@@ -357,6 +349,22 @@ void Server::rebuild(PinnedStage& stage)
 		{
 			j->group = load[1] < load[0] ? 1 : 0;
 			load[j->group] += 1ull << (j->spec.lx + j->spec.ly);
+		}
+	// SCABit lanes per row, for all rows of the tick alike
+	auto rowWords = [](const Job* j) { return j->spec.lx - (j->dev.wide ? 7 : 6); }; // log2
+	const int split = batch_row_split([&](int l) {
+		int64_t n = 0;
+		for(const Job* j : slots_)
+			if(runs(j) && j->dev.kind == BK_SCABIT)
+				n += 1ll << (j->spec.ly + std::min(rowWords(j), l));
+		return n;
+	});
+	for(Job* j : slots_)
+		if(runs(j) && j->dev.kind == BK_SCABIT)
+		{
+			const uint64_t du = j->dev.mode == 0 ? (j->dev.wide ? 2 : 1) : (j->dev.wide ? 64 : 32);
+			j->dev.lG = std::min(rowWords(j), split);
+			j->dev.stepJ = affine_pow(j->dev.step, du << j->dev.lG);
 		}
 	for(int g = 0; g < 2; ++g)
 	{
@@ -581,6 +589,7 @@ bool Server::enqueue(Tick& t)
 	}
 	const hipStream_t chain[2] = {s0_, s1_};
 	const bool two = nLanes_[1] > 0 || nWaves_[1] > 0;
+	const bool wave = nLanes_[0] + nLanes_[1] <= DT_WAVE_MAX_BLOCKS;
 	if(two)
 	{
 		check(hipEventRecord(fork_, s0_), "fork");
@@ -595,7 +604,7 @@ bool Server::enqueue(Tick& t)
 			for(int d = 0; d < 4 && da[c].nlanes > 0; ++d)
 			{
 				da[c].d = d;
-				check(launch_batch_dt(da[c], chain[c]), "batch_dt");
+				check(wave ? launch_batch_dt_wave(da[c], chain[c]) : launch_batch_dt(da[c], chain[c]), "batch_dt");
 			}
 			for(int s = 0; s < 2 && ca[c].nwaves > 0; ++s)
 			{
