@@ -21,7 +21,11 @@
 //
 // What bounds it: latency (the lattice and stream loads, the LDS round trips
 // of the level search, 20-24 dependent steps of 9 instructions) on small
-// lattices, VALU issue (about 700 instructions per block) from 4096^2 up.
+// lattices; from 4096^2 on VALU issue (about 700 instructions per block) and the
+// LDS (random 8-byte accesses, 28 per block and lane).  Tried and not kept: four
+// blocks per wave, levelled one after the other and applied together by 16
+// lanes each (4096^2 106 us per MCS against 91 then: twice the registers and
+// LDS).
 #include "kpz_kernels.hpp"
 
 namespace kpz {
@@ -33,7 +37,7 @@ constexpr int DW_PITCH = 17;                 // sites of a row and one empty col
 constexpr int DW_SITES = 18 * DW_PITCH;      // 16 rows with an empty row below and above
 constexpr int DW_LEVELS = 32;                // levels applied per pass
 constexpr int DW_LPITCH = DW_LEVELS + 4;     // words per row of the level table (16-byte aligned rows)
-static_assert(16 * DW_LPITCH * 4 <= 4 * DW_SITES * 8, "the level table reuses the window masks");
+static_assert(16 * DW_LPITCH * 4 <= 2 * DW_SITES * 8, "the level table reuses the window masks");
 
 // bits 0,2,..,30 -> 0..15
 __device__ __forceinline__ uint32_t even_bits(uint32_t v)
@@ -112,8 +116,8 @@ __device__ __forceinline__ void dt_wave_block(const DtPhaseArgs& a, const DtWave
 		// no update yet on any site of any window
 		uint4* z = reinterpret_cast<uint4*>(masks);
 #pragma unroll
-		for(int k = 0; k < (4 * DW_SITES * 8 / 16 + 63) / 64; ++k)
-			if(64 * k + lane < 4 * DW_SITES * 8 / 16)
+		for(int k = 0; k < (2 * DW_SITES * 8 / 16 + 63) / 64; ++k)
+			if(64 * k + lane < 2 * DW_SITES * 8 / 16)
 				z[64 * k + lane] = make_uint4(0, 0, 0, 0);
 	}
 
@@ -161,22 +165,34 @@ __device__ __forceinline__ void dt_wave_block(const DtPhaseArgs& a, const DtWave
 		s = J.window(s);
 	}
 
-	// ---- earlier updates of the window on the own or a neighbouring site
-	lds_in_order();
-#pragma unroll
-	for(int w = 0; w < 4; ++w)
-		if(live[w])
-			__hip_atomic_fetch_or(&masks[w * DW_SITES + at[w]], 1ull << lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-	lds_in_order();
+	// ---- earlier updates of the window on the own or a neighbouring site, two
+	// windows at a time (5 KB of LDS per wave, so that 8 waves fit a SIMD)
 	uint64_t before[4];
 	const uint64_t earlier = (1ull << lane) - 1;
-#pragma unroll
-	for(int w = 0; w < 4; ++w)
-	{
-		const uint64_t* m = masks + w * DW_SITES + at[w];
-		before[w] = (m[0] | m[-1] | m[1] | m[-DW_PITCH] | m[DW_PITCH]) & earlier;
-	}
 	lds_in_order();
+#pragma unroll
+	for(int w0 = 0; w0 < 4; w0 += 2)
+	{
+#pragma unroll
+		for(int k = 0; k < 2; ++k)
+			if(live[w0 + k])
+				__hip_atomic_fetch_or(&masks[k * DW_SITES + at[w0 + k]], 1ull << lane, __ATOMIC_RELAXED,
+				                      __HIP_MEMORY_SCOPE_WAVEFRONT);
+		lds_in_order();
+#pragma unroll
+		for(int k = 0; k < 2; ++k)
+		{
+			const uint64_t* m = masks + k * DW_SITES + at[w0 + k];
+			before[w0 + k] = (m[0] | m[-1] | m[1] | m[-DW_PITCH] | m[DW_PITCH]) & earlier;
+		}
+		lds_in_order();
+		if(w0 == 0)
+		{
+			masks[at[0]] = 0;
+			masks[DW_SITES + at[1]] = 0;
+			lds_in_order();
+		}
+	}
 
 	// ---- levels: an update waits while one of those has not been done
 	int level[4] = {0, 0, 0, 0}, depth[4] = {0, 0, 0, 0};
@@ -304,7 +320,7 @@ __device__ __forceinline__ void dt_wave_block(const DtPhaseArgs& a, const DtWave
 template<int UPD, bool RO>
 __global__ __launch_bounds__(64 * DW_WAVES) void dt_wave_kernel(DtPhaseArgs a, DtWaveJumps J, int64_t nb)
 {
-	__shared__ __align__(16) uint64_t masks[DW_WAVES][4 * DW_SITES];
+	__shared__ __align__(16) uint64_t masks[DW_WAVES][2 * DW_SITES];
 	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 	const int64_t i = (int64_t)blockIdx.x * DW_WAVES + wave;
 	if(i >= nb)
@@ -317,7 +333,7 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dt_wave_kernel(DtPhaseArgs a, D
 template<bool RO>
 __global__ __launch_bounds__(64 * DW_WAVES) void batch_dt_wave_kernel(BatchDtArgs a)
 {
-	__shared__ __align__(16) uint64_t masks[DW_WAVES][4 * DW_SITES];
+	__shared__ __align__(16) uint64_t masks[DW_WAVES][2 * DW_SITES];
 	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 	const int64_t e = (int64_t)blockIdx.x * DW_WAVES + wave + (RO ? a.nstatic : 0);
 	if(e >= (RO ? a.nlanes : a.nstatic))

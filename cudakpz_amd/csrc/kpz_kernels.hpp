@@ -52,10 +52,10 @@ struct DtWaveJumps {
 DtWaveJumps dt_wave_jumps(const Affine& step, int drawsPerUpdate);
 // Blocks up to which one wave per block is faster than one lane per block.
 // us per MCS (4 phases), lane / wave: 512^2 (2^8 blocks) KPZ 89 / 22, p/q 117 /
-// 21, disorder 175 / 24; 2048^2 (2^12) 91 / 34, 119 / 32, 177 / 40; 4096^2
-// (2^14) 93 / 91, 121 / 90, 180 / 113.  At 8192^2 (2^16) the wave kernel, bound
-// by instruction issue there, would take four times its 4096^2 figures and the
-// lane kernel 103, 140 and 228.
+// 20, disorder 175 / 25; 2048^2 (2^12) 91 / 33, 119 / 32, 177 / 44; 4096^2
+// (2^14) 93 / 80, 121 / 79, 180 / 115.  At 8192^2 (2^16) the wave kernel, bound
+// by instruction issue and the LDS there, would take four times its 4096^2
+// figures and the lane kernel 103, 140 and 221.
 constexpr int64_t DT_WAVE_MAX_BLOCKS = 1 << 14;
 // whether the phase takes less time with one wave per block than with one lane
 bool dt_wave_better(int lbx, int lby, int64_t nb, bool tinyMT);
