@@ -3125,6 +3125,244 @@ __global__ __launch_bounds__(256) void row_moments_kernel(const uint32_t* __rest
 	}
 }
 
+// Height moments by the 8-site walks, for rows of 64 sites and more.  Over 8
+// sites from height c the power sums are M_k = sum_j (c + p_j)^k, with the
+// walk's own sums P_k = sum_j p_j^k from a table and P_0 = 8: the transpose of
+// a polynomial's Taylor shift gives them in 28 multiply-adds (shift_moments).
+// A lane adds up the sums of its sites relative to its first one (whole numbers
+// below 2^53, so exact) and shifts them once per round to the true heights.
+// Per 8 sites 7 table reads and 35 fp64 operations, where the per-site loop
+// took 13 fp64 and some 9 integer operations a site: a moments() call at 16384^2
+// 363 -> 156 us, at 65536^2 3.63 -> 1.60 ms (ENC_CBBIT 3.40 -> 1.20); the
+// table reads (random 8-byte LDS accesses) bound it.
+constexpr int MOMENTS = 7;
+
+// M_k of values v -> of c + v (k = 0 .. MOMENTS)
+__device__ __forceinline__ void shift_moments(double (&M)[MOMENTS + 1], double c)
+{
+#pragma unroll
+	for(int i = MOMENTS - 1; i >= 0; --i)
+#pragma unroll
+		for(int k = i; k < MOMENTS; ++k)
+			M[k + 1] = __builtin_fma(c, M[k], M[k + 1]);
+}
+
+// site order of a table index: ENC_LOCAL bit 2k = site k, bit 2k + 1 = site
+// 4 + k (k < 4); ENC_CBBIT bit j = site 2j, bit 4 + j = site 2j + 1
+template<int ENC>
+__device__ __forceinline__ void build_moment_table(double (*tab)[256])
+{
+	const int i = threadIdx.x;
+	double P[MOMENTS];
+#pragma unroll
+	for(int e = 0; e < MOMENTS; ++e)
+		P[e] = 0;
+	int p = 0;
+#pragma unroll
+	for(int j = 0; j < 8; ++j)
+	{
+		p += corr_site_bit<ENC>((uint32_t)i, j) ? 1 : -1;
+		double q = p;
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+		{
+			P[e] += q;
+			q *= p;
+		}
+	}
+#pragma unroll
+	for(int e = 0; e < MOMENTS; ++e)
+		tab[e][i] = P[e];
+}
+
+// a lane's sums of powers of the heights relative to its first site's walk
+// start, and the walk's height so far
+struct LaneMoments {
+	double m[MOMENTS];
+	int c;
+	__device__ __forceinline__ void reset(int start)
+	{
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			m[e] = 0;
+		c = start;
+	}
+	__device__ __forceinline__ void chunk(const double (*tab)[256], uint32_t idx)
+	{
+		double M[MOMENTS + 1];
+		M[0] = 8.0;
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			M[e + 1] = tab[e][idx];
+		shift_moments(M, (double)c);
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			m[e] += M[e + 1];
+		c += 2 * __popc(idx) - 8;
+	}
+	// adds the lane's n sites, whose walk started at height h, to sum
+	__device__ __forceinline__ void add_to(double (&sum)[MOMENTS], double n, double h) const
+	{
+		double M[MOMENTS + 1];
+		M[0] = n;
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			M[e + 1] = m[e];
+		shift_moments(M, h);
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			sum[e] += M[e + 1];
+	}
+};
+
+// The walk of a row covers sites 1 .. L - 1 from the row's start height; site
+// 0 comes last, at start + D.  Lane 0 starts its walk at -s0 (s0 the slope at
+// x = 0), so that site 0 passes at relative height 0 and only its count is
+// taken out.
+__device__ __forceinline__ void finish_moments(double (&m)[MOMENTS], double h, int lane, double* __restrict__ out)
+{
+	double p = h; // site 0
+	if(lane == 0)
+	{
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+		{
+			m[e] += p;
+			p *= h;
+		}
+	}
+#pragma unroll
+	for(int e = 0; e < MOMENTS; ++e)
+	{
+#pragma unroll
+		for(int o = 32; o > 0; o >>= 1)
+			m[e] += __shfl_xor(m[e], o, 64);
+	}
+	if(lane == 0)
+	{
+#pragma unroll
+		for(int e = 0; e < MOMENTS; ++e)
+			out[e] = m[e];
+	}
+}
+
+// one wave per word row of four site rows, taken one after the other
+__global__ __launch_bounds__(256) void row_moments_local_kernel(const uint32_t* __restrict__ lat, int lx, int ly,
+		const int64_t* __restrict__ hs, double* __restrict__ out)
+{
+	__shared__ double tab[MOMENTS][256];
+	build_moment_table<ENC_LOCAL>(tab);
+	__syncthreads();
+	const int yw = blockIdx.x * 4 + (threadIdx.x >> 6);
+	const int lane = threadIdx.x & 63;
+	if(yw >= (1 << (ly - 2)))
+		return; // uniform per wave; no barrier below
+	const int XW = 1 << (lx - 2);
+	const int K = XW >= 64 * 8 ? 8 : (XW > 128 ? XW / 64 : 2); // words per lane and round
+	const uint32_t* __restrict__ row = lat + ((size_t)yw << (lx - 2));
+	for(int r = 0; r < 4; ++r)
+	{
+		const int64_t h0 = hs[4 * yw + r];
+		const int s0 = ((row[0] >> (8 * r)) & 1u) ? 1 : -1;
+		double sum[MOMENTS] = {0, 0, 0, 0, 0, 0, 0};
+		int64_t base = h0 - s0; // height before the round's first site
+		for(int w0 = 0; w0 < XW; w0 += 64 * K)
+		{
+			const int wl = w0 + lane * K;
+			const bool live = wl < XW, first = wl == 0;
+			LaneMoments L;
+			const int start = first ? -s0 : 0;
+			L.reset(start);
+			if(live)
+				for(int k = 0; k < K; k += 2)
+				{
+					const uint2 v = *reinterpret_cast<const uint2*>(row + wl + k);
+					L.chunk(tab, ((v.x >> (8 * r)) & 0x55u) | (((v.y << 1) >> (8 * r)) & 0xAAu));
+				}
+			const int q = L.c - start;
+			const int incl = wave_incl_scan32(q);
+			if(live)
+				L.add_to(sum, first ? 4.0 * K - 1.0 : 4.0 * K, (double)(base + (incl - q) - start));
+			base += wave_last32(incl);
+		}
+		finish_moments(sum, (double)(base + s0), lane, out + (size_t)(4 * yw + r) * MOMENTS);
+	}
+}
+
+__global__ __launch_bounds__(256) void row_moments_cbbit_kernel(const uint32_t* __restrict__ lat, int lx, int ly,
+		const int64_t* __restrict__ hs, double* __restrict__ out)
+{
+	__shared__ double tab[MOMENTS][256];
+	build_moment_table<ENC_CBBIT>(tab);
+	__syncthreads();
+	const int y = blockIdx.x * 4 + (threadIdx.x >> 6);
+	const int lane = threadIdx.x & 63;
+	if(y >= (1 << ly))
+		return; // uniform per wave; no barrier below
+	const int WR = 1 << (lx - 6); // words per row and quadrant
+	const size_t sw = (size_t)1 << (lx + ly - 4);
+	const size_t rowW = (size_t)y << (lx - 6);
+	const uint32_t* __restrict__ ev = lat + rowW + ((y & 1) ? (sw >> 1) : 0);
+	const uint32_t* __restrict__ od = lat + rowW + ((y & 1) ? 0 : (sw >> 1));
+	const int64_t h0 = hs[y];
+	const int s0 = (ev[0] & 1u) ? 1 : -1;
+	double sum[MOMENTS] = {0, 0, 0, 0, 0, 0, 0};
+	int64_t base = h0 - s0;
+	for(int w0 = 0; w0 < WR; w0 += 64)
+	{
+		const int wl = w0 + lane;
+		const bool live = wl < WR, first = wl == 0;
+		LaneMoments L;
+		const int start = first ? -s0 : 0;
+		L.reset(start);
+		if(live)
+		{
+			// as row_stats_cbbit_kernel
+			const uint32_t e = ev[wl], o = od[wl];
+			const uint32_t lo = __builtin_amdgcn_bitop3_b32(e, o << 4, 0x0F0F0F0Fu, 0xE4);
+			const uint32_t hi = __builtin_amdgcn_bitop3_b32(e >> 4, o, 0x0F0F0F0Fu, 0xE4);
+			for(int k = 0; k < 4; ++k)
+			{
+				L.chunk(tab, (lo >> (8 * k)) & 0xFFu);
+				L.chunk(tab, (hi >> (8 * k)) & 0xFFu);
+			}
+		}
+		const int q = L.c - start;
+		const int incl = wave_incl_scan32(q);
+		if(live)
+			L.add_to(sum, first ? 63.0 : 64.0, (double)(base + (incl - q) - start));
+		base += wave_last32(incl);
+	}
+	finish_moments(sum, (double)(base + s0), lane, out + (size_t)y * MOMENTS);
+}
+
+// The rows' sums, MOMENT_GROUP rows to one pair {value, rounding error} per
+// power (error-free additions, Knuth), for the host to add up
+constexpr int MOMENT_GROUP = 64;
+__global__ __launch_bounds__(64) void moments_group_kernel(const double* __restrict__ rows, int ny, double* __restrict__ out)
+{
+	const int lane = threadIdx.x;
+	const int y = blockIdx.x * MOMENT_GROUP + lane;
+#pragma unroll
+	for(int e = 0; e < MOMENTS; ++e)
+	{
+		double hi = (y < ny) ? rows[(size_t)y * MOMENTS + e] : 0.0, lo = 0.0;
+#pragma unroll
+		for(int o = 32; o > 0; o >>= 1)
+		{
+			const double b = __shfl_xor(hi, o, 64), bl = __shfl_xor(lo, o, 64);
+			const double s = hi + b, t = s - hi;
+			lo += bl + ((hi - (s - t)) + (b - t));
+			hi = s;
+		}
+		if(lane == 0)
+		{
+			out[((size_t)blockIdx.x * MOMENTS + e) * 2] = hi;
+			out[((size_t)blockIdx.x * MOMENTS + e) * 2 + 1] = lo;
+		}
+	}
+}
+
 // ---------------------------------------------------------------- fill
 __global__ void fill_kernel(uint32_t* lat, uint64_t n, uint64_t split, uint32_t lo, uint32_t hi)
 {
@@ -3780,14 +4018,22 @@ hipError_t launch_cbbit_half(const CbHalfArgs& a, hipStream_t stream)
 	return hipGetLastError();
 }
 
-hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, const int64_t* hs, double* out,
+int64_t moment_groups(int ly) { return (((int64_t)1 << ly) + MOMENT_GROUP - 1) / MOMENT_GROUP; }
+
+hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, const int64_t* hs, double* rows, double* groups,
 		hipStream_t stream)
 {
 	const dim3 grid((unsigned)(((1 << ly) + 3) / 4));
-	if(enc == ENC_LOCAL)
-		hipLaunchKernelGGL((row_moments_kernel<ENC_LOCAL>), grid, dim3(256), 0, stream, lat, lx, ly, hs, out);
+	if(enc == ENC_LOCAL && lx >= 6 && ly >= 2)
+		hipLaunchKernelGGL(row_moments_local_kernel, dim3((unsigned)(((1 << (ly - 2)) + 3) / 4)), dim3(256), 0, stream, lat,
+		                   lx, ly, hs, rows);
+	else if(enc == ENC_CBBIT && lx >= 6)
+		hipLaunchKernelGGL(row_moments_cbbit_kernel, grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
+	else if(enc == ENC_LOCAL)
+		hipLaunchKernelGGL((row_moments_kernel<ENC_LOCAL>), grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
 	else
-		hipLaunchKernelGGL((row_moments_kernel<ENC_CBBIT>), grid, dim3(256), 0, stream, lat, lx, ly, hs, out);
+		hipLaunchKernelGGL((row_moments_kernel<ENC_CBBIT>), grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
+	hipLaunchKernelGGL(moments_group_kernel, dim3((unsigned)moment_groups(ly)), dim3(64), 0, stream, rows, 1 << ly, groups);
 	return hipGetLastError();
 }
 

@@ -181,9 +181,11 @@ hipError_t launch_tmt_chunk_polys(const TmtOrbit* orb, int64_t T, int chunks, ui
 // out[y*ROW_STATS + k] = {S1, S2, D, sy0, S1', D', sy0', S11, tcs, 0}, the
 // primed values from `snap` (zero when snap is null).
 constexpr int ROW_STATS = 10;
-// out[y*7 + k-1] = sum over row y of h^k (double), k = 1..7, given the exact
-// start height hs[y] of every row
-hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, const int64_t* hs, double* out,
+// rows[y*7 + k-1] = sum over row y of h^k (double), k = 1..7, given the exact
+// start height hs[y] of every row; groups[(g*7 + k-1)*2] = {sum of 64 rows, its
+// rounding error} for g < moment_groups(ly)
+int64_t moment_groups(int ly);
+hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, const int64_t* hs, double* rows, double* groups,
 		hipStream_t stream);
 // consistency of a lattice (SchedulerService::consitencyCheck): rowOnes[y] +=
 // ones among row y's x slopes, colOnes[x] = ones among column x's y slopes,

@@ -333,12 +333,17 @@ const Affine* SchedulerService::upload(std::vector<Affine>& host, DevBuf& buf)
 // (row_stats), combined on the device in int128 (row_combine); heights follow
 // Correlator::set (kpz/correlator.cpp:37-106).  hs (optional) receives every
 // row's start height.
-Sums SchedulerService::totals(const uint32_t* snap, int64_t* hs)
+void SchedulerService::queueTotals(const uint32_t* snap, int64_t* hs)
 {
 	check(launch_row_stats(deviceLattice(), snap, enc_, size_.lx, size_.ly, rows_.as<int64_t>(), stream_), "row_stats");
 	check(launch_row_combine(rows_.as<int64_t>(), size_.lx, size_.ly, snap != nullptr, hs,
 	                         rows_.as<int64_t>() + (size_t)size_.dimY() * ROW_STATS, totals_.as<int64_t>(), stream_),
 	      "row_combine");
+}
+
+Sums SchedulerService::totals(const uint32_t* snap)
+{
+	queueTotals(snap, nullptr);
 	sync();
 	const volatile int64_t* const r = totals_.as<int64_t>(); // host memory, written by the kernel
 	Sums s;
@@ -353,7 +358,7 @@ Sums SchedulerService::totals(const uint32_t* snap, int64_t* hs)
 	return s;
 }
 
-Sums SchedulerService::roughness() { return totals(nullptr, nullptr); }
+Sums SchedulerService::roughness() { return totals(nullptr); }
 
 // counts of one lattice (device or snapshot), added to out[0..2]
 void SchedulerService::consistencyOf(const uint32_t* lat, int64_t out[3])
@@ -394,22 +399,22 @@ bool SchedulerService::consistencyCheck(bool full, int64_t out[3])
 
 void SchedulerService::moments(long double out[7])
 {
-	const size_t ny = (size_t)1 << size_.ly;
+	const size_t ny = (size_t)1 << size_.ly, ng = (size_t)moment_groups(size_.ly);
 	if(!rowStart_.get())
 	{
-		rowStart_.alloc(ny * 8);
 		rowMoments_.alloc(ny * 7 * 8);
+		groupMoments_.alloc(ng * 14 * 8);
+		rowStart_.alloc(ny * 8);
 	}
-	totals(nullptr, rowStart_.as<int64_t>()); // every row's exact start height, on the device
-	check(launch_row_moments(deviceLattice(), enc_, size_.lx, size_.ly, rowStart_.as<int64_t>(),
-			rowMoments_.as<double>(), stream_), "row_moments");
-	std::vector<double> m(ny * 7);
-	check(hipMemcpyAsync(m.data(), rowMoments_.get(), m.size() * 8, hipMemcpyDeviceToHost, stream_), "moments D2H");
+	queueTotals(nullptr, rowStart_.as<int64_t>()); // every row's exact start height, on the device
+	check(launch_row_moments(deviceLattice(), enc_, size_.lx, size_.ly, rowStart_.as<int64_t>(), rowMoments_.as<double>(),
+			groupMoments_.as<double>(), stream_), "row_moments");
 	sync();
+	const volatile double* const m = groupMoments_.as<double>(); // host memory, written by the kernel
 	long double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-	for(size_t y = 0; y < ny; ++y)
+	for(size_t g = 0; g < ng; ++g)
 		for(int k = 0; k < 7; ++k)
-			acc[k] += m[y * 7 + (size_t)k];
+			acc[k] += (long double)m[(g * 7 + (size_t)k) * 2] + (long double)m[(g * 7 + (size_t)k) * 2 + 1];
 	const long double N = (long double)size_.sites();
 	for(int k = 0; k < 7; ++k)
 		out[k] = acc[k] / N;
@@ -462,7 +467,7 @@ std::vector<SchedulerService::TagResult> SchedulerService::correlateAll()
 	return out;
 }
 
-Sums SchedulerService::correlateWith(const DevBuf& snap) { return totals(snap.as<uint32_t>(), nullptr); }
+Sums SchedulerService::correlateWith(const DevBuf& snap) { return totals(snap.as<uint32_t>()); }
 
 // ======================================================================
 SchedulerDT::SchedulerDT(int lx, int ly, const Params& p, bool randomOrigin)

@@ -215,9 +215,10 @@ protected:
 	// gives back memory that only makes calls faster; false if there is none
 	virtual bool dropSpare() { return false; }
 	Sums correlateWith(const DevBuf& snap);
-	Sums totals(const uint32_t* snap, int64_t* hs);
+	void queueTotals(const uint32_t* snap, int64_t* hs); // hs: every row's start height, or null
+	Sums totals(const uint32_t* snap);
 	DevBuf lat_, rows_, rowStart_, rowMoments_, check_;
-	PinnedBuf totals_;
+	PinnedBuf totals_, groupMoments_;
 	void consistencyOf(const uint32_t* lat, int64_t out[3]);
 	std::vector<Tag> tags_;
 	DevBuf st_[2];
