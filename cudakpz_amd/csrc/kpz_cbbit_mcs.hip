@@ -1,5 +1,5 @@
-// One whole bit-parallel SCABit MCS (both half-sweeps, mode 0 of
-// cbbit_half_kernel) in one pass over the lattice.
+// One whole SCABit MCS (both half-sweeps, modes 0 and 1 of cbbit_half_kernel)
+// in one pass over the lattice.
 //
 // The bit-parallel half-sweep is bound by memory: each of the two reads and
 // writes every word (1 byte per site update in all) for a few instructions per
@@ -8,7 +8,8 @@
 // read once and written once per MCS: 65536^2 takes 441 us (788 in two
 // half-sweeps), 4.9 TB/s, what a copy of that size reaches; 16384^2 25 us (45),
 // 8192^2 9.6 (15), and on small lattices one launch instead of two, 2048^2 4.9
-// (6.6).
+// (6.6).  The per-site rule gains where its own half-sweeps come close to the
+// memory rate (cbbit_mcs_better).
 //
 // Half-sweep s acts on the sites of sublattice s.  On row y it flips bits of
 // X_s(y), Y_s(y), X_o(y) and Y_o(y + 1) (o the other sublattice), each bit
@@ -21,6 +22,8 @@
 // bits that cross from word to word stay inside it.  Source and destination are
 // different lattices, since neighbouring bands read each other's rows.
 #include "kpz_kernels.hpp"
+
+#include "kpz_draws.hpp"
 
 namespace kpz {
 
@@ -189,7 +192,8 @@ __device__ __forceinline__ void store2(uint64_t* p, const Words& v)
 	*reinterpret_cast<ulonglong2*>(p) = make_ulonglong2(v.a, v.b);
 }
 
-template<bool MULTI>
+// NT: 0 = bit-parallel, else per site with 1 (q = 0) or 2 thresholds per draw
+template<int NT, bool MULTI>
 __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMcsArgs a)
 {
 	__shared__ uint32_t low[16], high[16]; // per wave: bits for the wave before / after
@@ -211,11 +215,31 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 	RowWorker wk(y, a.per, a.rem);
 	const bool single = a.per == 1 && a.rem == 0;
 	auto row = [&](int yy) { return (size_t)(yy & (Y - 1)) * Wn + w; };
-	auto random = [&](uint64_t start) {
+	// sites that flip if they are a minimum (p) or a maximum (q), from the
+	// row's stream start
+	struct Accept {
+		Words p, q;
+	};
+	auto accept = [&](uint64_t start) {
 		uint64_t u = J(start);
-		Words r;
-		r.a = vl3_word(u, step);
-		r.b = vl3_word(u, step);
+		Accept r{{0, 0}, {0, 0}};
+		if constexpr(NT == 0)
+		{
+			r.p.a = vl3_word(u, step);
+			r.p.b = vl3_word(u, step);
+		}
+		else
+		{
+			uint32_t lo = (uint32_t)u, h24 = (uint32_t)(u >> 32);
+#pragma unroll 1
+			for(int k = 0; k < 2; ++k) // the second word's draws follow the first one's
+			{
+				uint64_t pb = 0, qb = 0, none = 0;
+				cbbit_word_draws<uint64_t, NT>(lo, h24, step, a.tp, a.tq, 0, 0, pb, qb, none, none);
+				r.p = {r.p.b, pb};
+				r.q = {r.q.b, qb};
+			}
+		}
 		return r;
 	};
 	// first bit of the next lane / last bit of the lane before, within the wave
@@ -225,8 +249,14 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 		return Words{(v.a >> 1) | (v.b << 63), (v.b >> 1) | ((uint64_t)in << 63)};
 	};
 	auto left = [&](const Words& f, uint32_t in) { return Words{(f.a << 1) | in, (f.b << 1) | (f.a >> 63)}; };
-	auto flips = [&](const Words& x, const Words& v, const Words& xs, const Words& up, const Words& r) {
-		return Words{~(x.a | v.a) & xs.a & up.a & r.a, ~(x.b | v.b) & xs.b & up.b & r.b};
+	auto flips = [&](const Words& x, const Words& v, const Words& xs, const Words& up, const Accept& r) {
+		Words f{~(x.a | v.a) & xs.a & up.a & r.p.a, ~(x.b | v.b) & xs.b & up.b & r.p.b};
+		if constexpr(NT == 2)
+		{
+			f.a |= x.a & v.a & ~(xs.a | up.a) & r.q.a;
+			f.b |= x.b & v.b & ~(xs.b | up.b) & r.q.b;
+		}
+		return f;
 	};
 	auto flip = [&](Words& v, const Words& f) {
 		v.a ^= f.a;
@@ -293,7 +323,7 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 		// row y and of the second one on row y - 1 are in the same bit
 		fetch(i);
 		{
-			const Words f = flips(x0, v0, x1, v1up, random(s0));
+			const Words f = flips(x0, v0, x1, v1up, accept(s0));
 			flip(x0, f);
 			flip(v0, f);
 			flip(v1up, f);
@@ -301,7 +331,7 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 		}
 		if(i >= 2)
 		{
-			const Words f = flips(px1, pv1, px0, v0, random(start1));
+			const Words f = flips(px1, pv1, px0, v0, accept(start1));
 			flip(px1, f);
 			flip(pv1, f);
 			flip(v0, f);
@@ -328,13 +358,13 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 			}
 		}
 		fetch(i + 1);
-		const Words f0 = flips(x0, v0, right(x1, inX1), v1up, random(s0));
+		const Words f0 = flips(x0, v0, right(x1, inX1), v1up, accept(s0));
 		flip(x0, f0);
 		flip(v0, f0);
 		flip(v1up, f0);
 		Words f1{0, 0};
 		if(i >= 2)
-			f1 = flips(px1, pv1, right(px0, inX0), v0, random(start1));
+			f1 = flips(px1, pv1, right(px0, inX0), v0, accept(start1));
 		uint32_t inF0 = prev_bit(f0.b), inF1 = prev_bit(f1.b);
 		if constexpr(MULTI)
 		{
@@ -367,8 +397,10 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 // waves.  us per MCS with targets of 1024 / 2048 / 8192 waves (8192: at least 4
 // rows): 512^2 4.6 / 4.6 / 5.9, 4096^2 5.5 / 5.5 / 6.6, 8192^2 11.4 / 9.6 / 9.6,
 // 16384^2 24.1 / 24.8 / 27.6, 32768^2 127 / 115 / 125, 65536^2 443 / 441 / 446.
-int cbbit_mcs_band(int lx, int ly)
+int cbbit_mcs_band(int lx, int ly, int mode)
 {
+	if(mode == 1)
+		return ly < 5 ? ly : 5; // 65536^2: 962 us per MCS with 16 rows, 912 with 32, 923 with 64
 	int lR = ly < 6 ? ly : 6;
 	const int lanes = lx <= 13 ? lx - 7 : lx - 8; // log2 lanes per band
 	while(lR > 1 && ((1ll << (ly - lR + lanes)) >> 6) < 2048)
@@ -379,16 +411,25 @@ int cbbit_mcs_band(int lx, int ly)
 hipError_t launch_cbbit_mcs(const CbMcsArgs& a, hipStream_t stream)
 {
 	if(!a.src || !a.dst || a.src == a.dst || !a.wordJ || !a.rowJ || a.lx < 7 || a.lx > CBBIT_MCS_MAX_LX || a.ly < 1 ||
-	   a.ly > 30 || a.lR < 1 || a.lR > a.ly || a.T < 1 || a.per < 1)
+	   a.ly > 30 || a.lR < 1 || a.lR > a.ly || a.T < 1 || a.per < 1 || a.mode < 0 || a.mode > 1 ||
+	   (a.mode == 1 && a.lx < 15))
 		return hipErrorInvalidValue;
 	const int64_t bands = 1ll << (a.ly - a.lR);
 	const int lW = a.lx - 7;
-	if(lW <= 6)
+	const dim3 wide((unsigned)(lW == 7 ? (bands + 3) / 4 : bands)), lanes(lW == 7 ? 256u : 1u << (lW - 1));
+	if(a.mode == 1)
+	{
+		if(a.tq)
+			hipLaunchKernelGGL((cbbit_mcs_wide_kernel<2, true>), wide, lanes, 0, stream, a);
+		else
+			hipLaunchKernelGGL((cbbit_mcs_wide_kernel<1, true>), wide, lanes, 0, stream, a);
+	}
+	else if(lW <= 6)
 		hipLaunchKernelGGL(cbbit_mcs_narrow_kernel, dim3((unsigned)(((bands << lW) + 255) / 256)), dim3(256), 0, stream, a);
 	else if(lW == 7)
-		hipLaunchKernelGGL(cbbit_mcs_wide_kernel<false>, dim3((unsigned)((bands + 3) / 4)), dim3(256), 0, stream, a);
+		hipLaunchKernelGGL((cbbit_mcs_wide_kernel<0, false>), wide, lanes, 0, stream, a);
 	else
-		hipLaunchKernelGGL(cbbit_mcs_wide_kernel<true>, dim3((unsigned)bands), dim3(1u << (lW - 1)), 0, stream, a);
+		hipLaunchKernelGGL((cbbit_mcs_wide_kernel<0, true>), wide, lanes, 0, stream, a);
 	return hipGetLastError();
 }
 

@@ -98,10 +98,19 @@ struct CbHalfArgs {
 };
 hipError_t launch_cbbit_half(const CbHalfArgs& a, hipStream_t stream);
 
-// ---- SCABit: both bit-parallel half-sweeps (mode 0) of an MCS in one pass ----
+// ---- SCABit: both half-sweeps of an MCS in one pass (modes 0 and 1) ----------
 // (kpz_cbbit_mcs.hip), from one lattice into another; lx >= 7
 constexpr int CBBIT_MCS_MAX_LX = 18; // a row is a workgroup of 1024 lanes then
-int cbbit_mcs_band(int lx, int ly);  // log2 rows of a band
+int cbbit_mcs_band(int lx, int ly, int mode); // log2 rows of a band
+// Whether MCS of `mode` are faster in one pass.  The per-site rule is bound by
+// VALU issue with the memory close behind (4.3 TB/s in two half-sweeps): one
+// pass pays from 2^31 sites on, where its bands of 32 rows fill the chip.  us per
+// MCS in half-sweeps / one pass, p = .95 q = .05 and q = 0: 65536^2 1021 / 912,
+// 890 / 761; 65536 x 32768 542 / 505, 471 / 414; 32768^2 294 / 301, 237 / 254.
+inline bool cbbit_mcs_better(int lx, int ly, int mode)
+{
+	return lx >= 7 && lx <= CBBIT_MCS_MAX_LX && (mode == 0 || (mode == 1 && lx >= 15 && lx + ly >= 31));
+}
 struct CbMcsArgs {
 	const uint32_t* src;
 	uint32_t* dst;
@@ -112,6 +121,8 @@ struct CbMcsArgs {
 	const Affine* rowJ;
 	const Affine* wordJ;    // wordJ[w]: skip w words of draws, all words of a row
 	Affine step, fullBig, fullSmall;
+	int mode;               // as CbHalfArgs
+	uint32_t tp, tq;
 	int lR;                 // log2 rows of a band
 };
 hipError_t launch_cbbit_mcs(const CbMcsArgs& a, hipStream_t stream);

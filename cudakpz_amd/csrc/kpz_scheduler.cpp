@@ -658,40 +658,45 @@ SchedulerSCABit::Tables& SchedulerSCABit::tables(int mode)
 	return ref;
 }
 
-// Whether bit-parallel MCS run in one pass (kpz_cbbit_mcs.hip), for which the
+// Whether MCS of this mode run in one pass (kpz_cbbit_mcs.hip), for which the
 // scheduler keeps a second lattice.  It is taken only for lattices of at most
 // 4 GiB and only while three quarters of the device's memory stay free, so that
 // programs that fill the memory with lattices or tags find it as before.
-bool SchedulerSCABit::wholeMcs()
+bool SchedulerSCABit::wholeMcs(int mode)
 {
-	if(wholeMcs_ != UNKNOWN)
-		return wholeMcs_ == YES;
-	wholeMcs_ = NO;
-	const size_t bytes = (size_t)size_.sizeW() * 4;
-	if(size_.lx < 7 || size_.lx > CBBIT_MCS_MAX_LX || bytes > ((size_t)4 << 30))
+	if(altState_ == NO || !cbbit_mcs_better(size_.lx, size_.ly, mode))
 		return false;
-	size_t free = 0, total = 0;
-	if(hipMemGetInfo(&free, &total) != hipSuccess || free < bytes || free - bytes < total / 4 * 3)
-		return false;
-	try
+	if(altState_ == UNKNOWN)
 	{
-		alt_.alloc(bytes);
+		altState_ = NO;
+		const size_t bytes = (size_t)size_.sizeW() * 4;
+		size_t free = 0, total = 0;
+		if(bytes > ((size_t)4 << 30) || hipMemGetInfo(&free, &total) != hipSuccess || free < bytes ||
+		   free - bytes < total / 4 * 3)
+			return false;
+		try
+		{
+			alt_.alloc(bytes);
+		}
+		catch(const Error&)
+		{
+			(void)hipGetLastError();
+			return false;
+		}
+		altState_ = YES;
 	}
-	catch(const Error&)
+	if(!wordJ_[mode].get())
 	{
-		(void)hipGetLastError();
-		return false;
+		std::vector<Affine> word((size_t)1 << (size_.lx - 7));
+		const Affine wordStep = affine_pow(step_, mode == 0 ? 2 : 64);
+		Affine acc{1, 0};
+		for(auto& j : word)
+		{
+			j = acc;
+			acc = compose(wordStep, acc);
+		}
+		upload(word, wordJ_[mode]);
 	}
-	std::vector<Affine> word((size_t)1 << (size_.lx - 7));
-	const Affine wordStep = affine_pow(step_, 2);
-	Affine acc{1, 0};
-	for(auto& j : word)
-	{
-		j = acc;
-		acc = compose(wordStep, acc);
-	}
-	upload(word, wordJ_);
-	wholeMcs_ = YES;
 	return true;
 }
 
@@ -701,7 +706,7 @@ bool SchedulerSCABit::dropSpare()
 		return false;
 	sync();
 	alt_.alloc(0);
-	wholeMcs_ = NO;
+	altState_ = NO;
 	return true;
 }
 
@@ -792,7 +797,7 @@ void SchedulerSCABit::run(int n, int mode)
 	a.tq = thresh23(q_);
 	a.lG = lG_;
 	// (asked for on any first call: later ones may be under capture)
-	if(mode == 0 && wholeMcs())
+	if(mode <= 1 && wholeMcs(mode))
 	{
 		// pairs of whole MCS, so that the lattice stays where it is
 		CbMcsArgs w{};
@@ -802,11 +807,14 @@ void SchedulerSCABit::run(int n, int mode)
 		w.per = per_;
 		w.rem = rem_;
 		w.rowJ = a.rowJ;
-		w.wordJ = wordJ_.as<Affine>();
+		w.wordJ = wordJ_[mode].as<Affine>();
+		w.mode = mode;
+		w.tp = a.tp;
+		w.tq = a.tq;
 		w.step = step_;
 		w.fullBig = a.fullBig;
 		w.fullSmall = a.fullSmall;
-		w.lR = cbbit_mcs_band(size_.lx, size_.ly);
+		w.lR = cbbit_mcs_band(size_.lx, size_.ly, mode);
 		for(; n >= 2; n -= 2)
 			for(int k = 0; k < 2; ++k)
 			{

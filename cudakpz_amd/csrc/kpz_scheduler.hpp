@@ -289,14 +289,14 @@ private:
 	};
 	void run(int n, int mode);
 	Tables& tables(int mode);
-	bool wholeMcs();
+	bool wholeMcs(int mode);
 	bool dropSpare() override;
 	int per_, rem_, lG_;
 	std::map<int, std::unique_ptr<Tables>> tab_;
-	// bit-parallel MCS in one pass: the other lattice and the jumps to every word
-	// of a row; wholeMcs_: not asked for yet, in use, not to be had
-	DevBuf alt_, wordJ_;
-	enum { UNKNOWN, YES, NO } wholeMcs_ = UNKNOWN;
+	// MCS in one pass: the other lattice and, per mode, the jumps to every word of
+	// a row; alt_ not asked for yet, in use, not to be had
+	DevBuf alt_, wordJ_[2];
+	enum { UNKNOWN, YES, NO } altState_ = UNKNOWN;
 };
 
 // Checkerboard SCA on ENC_LOCAL: SchedulerCPUCB semantics (the CPU

@@ -64,3 +64,19 @@ def test_pq_at_half():
     O.cbbit_mcs(lat, 15, 6, st, 2, 0)
     assert np.array_equal(s.popSystem(), lat)
     assert np.array_equal(s.streams(), st.states)
+
+
+# the per-site rule takes one pass from 2^31 sites on (512 MiB)
+@pytest.mark.parametrize("lx,ly,T,p,q", [(18, 13, 37, 0.7, 0.0), (15, 16, 0, 0.95, 0.05)])
+def test_per_site_in_one_pass(lx, ly, T, p, q):
+    s = K.SchedulerSCABit(lx, ly, threads=T)
+    s.supplySeed(31)
+    s.initHomogeneous()
+    s.setPQ(p, q)
+    s.mcsPQSyncRng(3)
+    m = O.Dsfmt(O.seed32(31))
+    st = O.Streams(s.threads, m)
+    lat = O.flat(lx, ly, O.ENC_CBBIT)
+    O.cbbit_mcs_threaded(lat, lx, ly, st, 3, 1, p, q, THREADS)
+    assert np.array_equal(s.popSystem(), lat)
+    assert np.array_equal(s.streams(), st.states)
