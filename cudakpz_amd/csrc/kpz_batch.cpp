@@ -361,6 +361,7 @@ Batch::Chunk& Batch::graphFor(int b, int len)
 		da.nreps = size();
 		da.nlanes = dtLanes_[g];
 		da.nstatic = dtStatic_[g];
+		da.together = dtLanes_[0] + dtLanes_[1];
 	}
 	const bool wave = dtLanes_[0] + dtLanes_[1] <= DT_WAVE_MAX_BLOCKS;
 	BatchCbArgs cg[2];

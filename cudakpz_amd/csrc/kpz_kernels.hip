@@ -59,6 +59,15 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t v, int src, int width)
 
 __device__ __forceinline__ uint32_t shflw(uint32_t v, int src, int width) { return (uint32_t)__shfl((int)v, src, width); }
 
+// v + v as v_add_u32: left shifts issue at half the rate of adds on gfx950,
+// and the compiler turns v + v written in C into a shift
+__device__ __forceinline__ uint32_t twice(uint32_t v)
+{
+	uint32_t r;
+	asm("v_add_u32 %0, %1, %1" : "=v"(r) : "v"(v));
+	return r;
+}
+
 // ======================================================================
 // DT phase kernel
 // ======================================================================
@@ -346,15 +355,6 @@ __device__ __forceinline__ void dt_writeback_x16s(uint32_t* __restrict__ lat, in
 // planes of T words: status[0..3], mat1, mat2, tmat (the layout of
 // TinyMT32::d_Random, kpz/GPUTinyMT.cu:38-61, and of its `.tinyMT` dataset).
 // ======================================================================
-// v + v as v_add_u32: left shifts issue at half the rate of adds on gfx950,
-// and the compiler turns v + v written in C into a shift
-__device__ __forceinline__ uint32_t twice(uint32_t v)
-{
-	uint32_t r;
-	asm("v_add_u32 %0, %1, %1" : "=v"(r) : "v"(v));
-	return r;
-}
-
 struct TinyMT {
 	uint32_t s0, s1, s2, s3, m1, m2, tm;
 
@@ -507,8 +507,13 @@ struct DtTmt {
 // the stream cursor `cur`.  nb = blocks per domain set.  UPD: 0 = KPZ
 // (pqOneUpdate), 1 = pqSyncRngUpdate, 2 = disorder2SyncRngUpdate (class rows
 // of the disorder map in myD, 2 bits per site), 3 = EW.
-// RUNS: the draws of several updates in one run (below).
-template<int LBX, int LBY, int UPD, bool RO, bool RUNS, class Cur>
+// LOOP: when an update's draws are taken (dt_launch and launch_batch_dt choose).
+enum DtLoop {
+	PLAIN, // before it
+	AHEAD, // behind the LDS reads of the update before it
+	RUNS   // those of four updates in one run (draws_begin)
+};
+template<int LBX, int LBY, int UPD, bool RO, DtLoop LOOP, class Cur>
 __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_t nb, const DtTile& my,
                                          uint32_t* __restrict__ myD, Cur& cur)
 {
@@ -621,8 +626,8 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 
 	// ---- BX*BY random-sequential updates (Func_MCSBase::exec,
 	// kpz/schedulerCPUDT_nested.h:46-66; pqOneUpdate kpz/schedulerCPU.inl:21-33)
-	constexpr bool ACCEPT = UPD == 1 || UPD == 2; // an acceptance draw per update
-	auto update = [&](uint32_t d1, uint32_t d2, uint32_t d3) {
+	// behindReads: what to do while the LDS reads are on their way
+	auto update = [&](uint32_t d1, uint32_t d2, uint32_t d3, auto&& behindReads) {
 		// x comes as xr = (BX - 1) - x, the same bits of ~r1 (one v_xnor_b32 with
 		// the fold), so that the column mask 1 << x is a right shift: right
 		// shifts issue at twice the rate of left shifts
@@ -648,6 +653,7 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 		const uint32_t cm = (1u << (BX - 1)) >> xr; // 1 << x
 		uint2 row = make_uint2(my.template Xb<BY>(yo), my.template Yb<BY>(yo));
 		const uint32_t up = my.template Yb<BY>(yo + DT_WG * 4);
+		behindReads();
 		// whole-row bit algebra, then select column x: a local minimum has
 		// own X = 0, right X = 1, own Y = 0, up Y = 1; a maximum the opposite
 		const uint32_t rx = row.x >> 1;
@@ -680,19 +686,33 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 				aMin = (uint32_t)((int32_t)(r23 - tpv) >> 31);
 				aMax = (uint32_t)((int32_t)(r23 - tqv) >> 31);
 			}
-			const uint32_t mn = rx & ~row.x & ~row.y & up;
-			const uint32_t mx = ~rx & row.x & row.y & ~up;
-			// a minimum flips as X - m (bit x set, bit x+1 cleared), a maximum
-			// as X + m (the opposite); Y and the Y above toggle either way
-			const uint32_t fn = mn & aMin & cm, fx = mx & aMax & cm;
-			my.template setXb<BY>(yo, row.x - fn + fx);
-			my.template setYb<BY>(yo, row.y ^ fn ^ fx);
-			my.template setYb<BY>(yo + DT_WG * 4, up ^ fn ^ fx);
+			if constexpr(LOOP == RUNS)
+			{
+				// two instructions less, in a longer chain (DT_RUNS_MIN_LANES): an
+				// extremum has own X = own Y, both different from right X and up Y,
+				// and is a minimum where they are 0; a flip exchanges the x slopes x
+				// and x + 1 and the y slopes of the row and the one above
+				const uint32_t ext = (row.x ^ rx) & ~(row.x ^ row.y) & (row.y ^ up);
+				const uint32_t f = ext & ((row.x & aMax) | (~row.x & aMin)) & cm;
+				my.template setXb<BY>(yo, row.x ^ f ^ twice(f));
+				my.template setYb<BY>(yo, row.y ^ f);
+				my.template setYb<BY>(yo + DT_WG * 4, up ^ f);
+			}
+			else
+			{
+				const uint32_t mn = rx & ~row.x & ~row.y & up;
+				const uint32_t mx = ~rx & row.x & row.y & ~up;
+				// a minimum flips as X - m (bit x set, bit x+1 cleared), a maximum
+				// as X + m (the opposite); Y and the Y above toggle either way
+				const uint32_t fn = mn & aMin & cm, fx = mx & aMax & cm;
+				my.template setXb<BY>(yo, row.x - fn + fx);
+				my.template setYb<BY>(yo, row.y ^ fn ^ fx);
+				my.template setYb<BY>(yo + DT_WG * 4, up ^ fn ^ fx);
+			}
 		}
 	};
-	if constexpr(RUNS)
+	if constexpr(LOOP == RUNS)
 	{
-		// the 12 draws of 4 updates in one run (draws_begin); dt_launch says when
 		constexpr int U = 4;
 #pragma unroll 1
 		for(int k = 0; k < BX * BY; k += U)
@@ -705,18 +725,41 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 			draws_end();
 #pragma unroll
 			for(int u = 0; u < U; ++u)
-				update(d[3 * u], d[3 * u + 1], d[3 * u + 2]);
+				update(d[3 * u], d[3 * u + 1], d[3 * u + 2], [] {});
 		}
 	}
 	else
 	{
-#pragma unroll 2
-		for(int k = 0; k < BX * BY; ++k)
+		constexpr bool ACCEPT = UPD == 1 || UPD == 2; // an acceptance draw per update
+		if constexpr(LOOP == AHEAD)
 		{
-			const uint32_t d1 = cur.draw();
-			const uint32_t d2 = cur.draw();
-			const uint32_t d3 = ACCEPT ? cur.draw() : 0u;
-			update(d1, d2, d3);
+			uint32_t d[3] = {0, 0, 0};
+			auto draw = [&] {
+				d[0] = cur.draw();
+				d[1] = cur.draw();
+				if(ACCEPT)
+					d[2] = cur.draw();
+			};
+			draw();
+#pragma unroll 2
+			for(int k = 0; k < BX * BY - 1; ++k)
+				update(d[0], d[1], d[2], [&] {
+					__builtin_amdgcn_sched_barrier(0);
+					draw();
+					__builtin_amdgcn_sched_barrier(0);
+				});
+			update(d[0], d[1], d[2], [] {});
+		}
+		else
+		{
+#pragma unroll 2
+			for(int k = 0; k < BX * BY; ++k)
+			{
+				const uint32_t d1 = cur.draw();
+				const uint32_t d2 = cur.draw();
+				const uint32_t d3 = ACCEPT ? cur.draw() : 0u;
+				update(d1, d2, d3, [] {});
+			}
 		}
 	}
 
@@ -767,7 +810,7 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 	}
 }
 
-template<int LBX, int LBY, int UPD, bool RO, bool RUNS>
+template<int LBX, int LBY, int UPD, bool RO, DtLoop LOOP>
 __global__ __launch_bounds__(DT_WG) void dt_phase_kernel(DtPhaseArgs a, int64_t nb)
 {
 	// X plane then Y plane in one array: both planes share one address
@@ -778,7 +821,7 @@ __global__ __launch_bounds__(DT_WG) void dt_phase_kernel(DtPhaseArgs a, int64_t 
 	if(i >= nb)
 		return; // no barrier in this kernel: idle lanes may leave
 	DtSlcg<RO> cur;
-	dt_block<LBX, LBY, UPD, RO, RUNS>(a, i, nb,
+	dt_block<LBX, LBY, UPD, RO, LOOP>(a, i, nb,
 	                            DtTile{tile + threadIdx.x, tile + (1 << LBY) * DT_WG + threadIdx.x, tile, threadIdx.x * 4},
 	                            (UPD == 2) ? tileD + threadIdx.x : nullptr, cur);
 }
@@ -807,7 +850,7 @@ __global__ __launch_bounds__(DT_WG) void dt_tmt_kernel(DtPhaseArgs a, int64_t nb
 		if(c >= nb)
 			return; // no barrier in this kernel; workers without a block keep their stream
 		cur.g = TinyMT::load(g, a.T, c);
-		dt_block<LBX, LBY, UPD, true, false>(a, c, nb, my, myD, cur);
+		dt_block<LBX, LBY, UPD, true, UPD == 2 ? PLAIN : AHEAD>(a, c, nb, my, myD, cur);
 		cur.g.store(g, a.T, c);
 		return;
 	}
@@ -828,7 +871,7 @@ __global__ __launch_bounds__(DT_WG) void dt_tmt_kernel(DtPhaseArgs a, int64_t nb
 	}
 	for(int m = 0; m < C && i < nb; ++m, i += a.T)
 	{
-		dt_block<LBX, LBY, UPD, true, false>(a, i, nb, my, myD, cur);
+		dt_block<LBX, LBY, UPD, true, UPD == 2 ? PLAIN : AHEAD>(a, i, nb, my, myD, cur);
 		if(i + a.T >= nb)
 			cur.g.store(a.tmtOut, a.T, t);
 	}
@@ -3338,7 +3381,8 @@ __global__ __launch_bounds__(256) void copy_kernel(uint4* __restrict__ dst, cons
 // RO: the DTr lanes [nstatic, nlanes), else the static DT lanes [0, nstatic):
 // one kernel per kind, so that the static DT lanes keep the register budget
 // (and occupancy) of the static update loop rather than the DTr staging's
-template<bool RO>
+// PQ: the loop of the p/q rule (DT_RUNS_MIN_LANES)
+template<bool RO, DtLoop PQ>
 __global__ __launch_bounds__(DT_WG) void batch_dt_kernel(BatchDtArgs a)
 {
 	__shared__ uint32_t tile[33 * DT_WG]; // X plane (16 rows), Y plane (17 rows)
@@ -3374,18 +3418,18 @@ __global__ __launch_bounds__(DT_WG) void batch_dt_kernel(BatchDtArgs a)
 		p.sy = sh >> 8;
 		DtSlcg<true> cur;
 		if(rep.mode)
-			dt_block<4, 4, 1, true, false>(p, w.y, nb, my, nullptr, cur);
+			dt_block<4, 4, 1, true, PQ>(p, w.y, nb, my, nullptr, cur);
 		else
-			dt_block<4, 4, 0, true, false>(p, w.y, nb, my, nullptr, cur);
+			dt_block<4, 4, 0, true, PLAIN>(p, w.y, nb, my, nullptr, cur);
 	}
 	else
 	{
 		p.sx = p.sy = 0;
 		DtSlcg<false> cur;
 		if(rep.mode)
-			dt_block<4, 4, 1, false, false>(p, w.y, nb, my, nullptr, cur);
+			dt_block<4, 4, 1, false, PQ>(p, w.y, nb, my, nullptr, cur);
 		else
-			dt_block<4, 4, 0, false, false>(p, w.y, nb, my, nullptr, cur);
+			dt_block<4, 4, 0, false, PLAIN>(p, w.y, nb, my, nullptr, cur);
 	}
 }
 
@@ -3637,32 +3681,45 @@ __global__ __launch_bounds__(BC_WG) void batch_combine_kernel(const BatchRep* __
 	}
 }
 
-// Lanes from which the p/q rule draws in runs of 12 (draws_begin): it pays
-// where several waves share a SIMD.  ms per MCS, p = q = .5, without and with
-// the runs, static and random origin: 8192^2 (2^16 lanes, a wave per SIMD)
-// 0.140 / 0.147 and 0.156 / 0.191; 16384^2 (2^18) 0.310 / 0.276 and 0.305 /
-// 0.274; 32768^2 1.09 / 0.98 and 0.98 / 0.94; 65536^2 4.08 / 3.73.  The
-// disorder rule loses with them (16384^2 0.52 / 0.56), and the rules of two
-// draws gain nothing (65536^2 2.65 / 2.67): their LDS accesses, 7.7 ns per wave
-// and update, bound the chip to 2.1 T updates/s.
+// Lanes from which the p/q rule draws in runs of 12 (draws_begin) and takes the
+// shorter but more serial update: it pays where several waves share a SIMD.  ms
+// per MCS, p = q = .5, without and with, static and random origin: 8192^2 (2^16
+// lanes, a wave per SIMD) 0.139 / 0.149 and 0.156 / 0.174; 16384^2 (2^18) 0.310
+// / 0.266 and 0.304 / 0.265; 65536^2 4.08 / 3.65 and 3.74 / 3.48; a batch of
+// 1024 replicas, half of its DT blocks p/q, 6.00 / 5.83.  The disorder rule
+// loses with the runs (16384^2 0.52 / 0.56), and the rules of two draws gain
+// nothing (65536^2 2.65 / 2.67): their LDS accesses, 7.7 ns per wave and update,
+// bound the chip to 2.1 T updates/s.
 constexpr int64_t DT_RUNS_MIN_LANES = 1 << 18;
+// The other loops draw an update's numbers behind the LDS reads of the one
+// before it, which shortens the chain of a lane: us per MCS without / with,
+// 8192^2 KPZ 104 / 90, random origin 122 / 110, p/q 139 / 121 and 156 / 140;
+// 16384^2 208 / 202, 219 / 209; 65536^2 random origin 2797 / 2686.  Static KPZ
+// on 65536^2, bound by LDS and issue, does not gain (2717 / 2740), and the
+// disorder rule loses (8192^2 229 / 247).
+constexpr int64_t DT_PLAIN_MIN_LANES = 1 << 20;
 template<int LBX, int LBY, int UPD>
 void dt_launch(const DtPhaseArgs& a, int64_t nb, dim3 grid, hipStream_t stream)
 {
 	if(a.tmt)
 		hipLaunchKernelGGL((dt_tmt_kernel<LBX, LBY, UPD>), grid, dim3(DT_WG), 0, stream, a, nb, a.tmt);
-	else if(UPD == 1 && nb >= DT_RUNS_MIN_LANES)
-	{
-		constexpr bool RUNS = UPD == 1;
-		if(a.random_origin)
-			hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, true, RUNS>), grid, dim3(DT_WG), 0, stream, a, nb);
-		else
-			hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, false, RUNS>), grid, dim3(DT_WG), 0, stream, a, nb);
-	}
 	else if(a.random_origin)
-		hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, true, false>), grid, dim3(DT_WG), 0, stream, a, nb);
+	{
+		if(UPD == 1 && nb >= DT_RUNS_MIN_LANES)
+			hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, true, UPD == 1 ? RUNS : AHEAD>), grid, dim3(DT_WG), 0, stream, a,
+			                   nb);
+		else
+			hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, true, UPD == 2 ? PLAIN : AHEAD>), grid, dim3(DT_WG), 0, stream,
+			                   a, nb);
+	}
+	else if(UPD == 1 && nb >= DT_RUNS_MIN_LANES)
+		hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, false, UPD == 1 ? RUNS : AHEAD>), grid, dim3(DT_WG), 0, stream, a,
+		                   nb);
+	else if(UPD == 2 || nb >= DT_PLAIN_MIN_LANES)
+		hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, false, PLAIN>), grid, dim3(DT_WG), 0, stream, a, nb);
 	else
-		hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, false, false>), grid, dim3(DT_WG), 0, stream, a, nb);
+		hipLaunchKernelGGL((dt_phase_kernel<LBX, LBY, UPD, false, UPD == 2 ? PLAIN : AHEAD>), grid, dim3(DT_WG), 0, stream, a,
+		                   nb);
 }
 
 template<int LBX, int LBY>
@@ -4137,12 +4194,22 @@ hipError_t launch_batch_dt(const BatchDtArgs& a, hipStream_t stream)
 {
 	if(a.nstatic < 0 || a.nstatic > a.nlanes)
 		return hipErrorInvalidValue;
-	if(a.nstatic > 0)
-		hipLaunchKernelGGL(batch_dt_kernel<false>, dim3((unsigned)((a.nstatic + DT_WG - 1) / DT_WG)), dim3(DT_WG), 0,
-		                   stream, a);
-	if(a.nlanes > a.nstatic)
-		hipLaunchKernelGGL(batch_dt_kernel<true>, dim3((unsigned)((a.nlanes - a.nstatic + DT_WG - 1) / DT_WG)),
-		                   dim3(DT_WG), 0, stream, a);
+	const dim3 gridS((unsigned)((a.nstatic + DT_WG - 1) / DT_WG));
+	const dim3 gridR((unsigned)((a.nlanes - a.nstatic + DT_WG - 1) / DT_WG));
+	if(a.together >= DT_RUNS_MIN_LANES)
+	{
+		if(a.nstatic > 0)
+			hipLaunchKernelGGL((batch_dt_kernel<false, RUNS>), gridS, dim3(DT_WG), 0, stream, a);
+		if(a.nlanes > a.nstatic)
+			hipLaunchKernelGGL((batch_dt_kernel<true, RUNS>), gridR, dim3(DT_WG), 0, stream, a);
+	}
+	else
+	{
+		if(a.nstatic > 0)
+			hipLaunchKernelGGL((batch_dt_kernel<false, AHEAD>), gridS, dim3(DT_WG), 0, stream, a);
+		if(a.nlanes > a.nstatic)
+			hipLaunchKernelGGL((batch_dt_kernel<true, AHEAD>), gridR, dim3(DT_WG), 0, stream, a);
+	}
 	return hipGetLastError();
 }
 

@@ -253,6 +253,7 @@ struct BatchDtArgs {
 	int64_t nlanes;
 	int64_t nstatic;        // lanes [0, nstatic) hold static DT replicas, the rest DTr
 	                        // (the tables put static DT first, padded to whole waves)
+	int64_t together;       // lanes of all launches that run at the same time
 	int m, d;               // MCS within the chunk, position in the domain order
 	const int* limit;       // optional [r]: replica r only runs MCS m < limit[r]
 };

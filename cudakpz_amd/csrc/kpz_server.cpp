@@ -580,6 +580,7 @@ bool Server::enqueue(Tick& t)
 		da[c].nreps = maxSlots_;
 		da[c].nlanes = nLanes_[c];
 		da[c].nstatic = nStatic_[c];
+		da[c].together = nLanes_[0] + nLanes_[1];
 		da[c].limit = limitBuf_.as<int>();
 		ca[c] = BatchCbArgs{};
 		ca[c].reps = repTable_.as<BatchRep>();
