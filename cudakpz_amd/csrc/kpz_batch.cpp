@@ -363,7 +363,7 @@ Batch::Chunk& Batch::graphFor(int b, int len)
 		da.nstatic = dtStatic_[g];
 		da.together = dtLanes_[0] + dtLanes_[1];
 	}
-	const bool wave = dtLanes_[0] + dtLanes_[1] <= DT_WAVE_MAX_BLOCKS;
+	const bool wave = dtLanes_[0] + dtLanes_[1] <= DT_BATCH_WAVE_MAX_BLOCKS;
 	BatchCbArgs cg[2];
 	for(int g = 0; g < 2; ++g)
 	{

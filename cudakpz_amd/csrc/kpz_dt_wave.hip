@@ -388,9 +388,9 @@ void launch(const DtPhaseArgs& a, const DtWaveJumps& J, int64_t nb, hipStream_t 
 
 } // namespace
 
-bool dt_wave_better(int lbx, int lby, int64_t nb, bool tinyMT)
+bool dt_wave_better(int lbx, int lby, int64_t nb, int upd, bool tinyMT)
 {
-	return lbx == 4 && lby == 4 && !tinyMT && nb <= DT_WAVE_MAX_BLOCKS;
+	return lbx == 4 && lby == 4 && !tinyMT && nb <= (upd == 2 ? 1 << 14 : 1 << 13);
 }
 
 DtWaveJumps dt_wave_jumps(const Affine& step, int drawsPerUpdate)

@@ -50,15 +50,15 @@ struct DtWaveJumps {
 	Affine window;   // J(64 draws per update): its next one
 };
 DtWaveJumps dt_wave_jumps(const Affine& step, int drawsPerUpdate);
-// Blocks up to which one wave per block is faster than one lane per block.
-// us per MCS (4 phases), lane / wave: 512^2 (2^8 blocks) KPZ 89 / 22, p/q 117 /
-// 20, disorder 175 / 25; 2048^2 (2^12) 91 / 33, 119 / 32, 177 / 44; 4096^2
-// (2^14) 93 / 80, 121 / 79, 180 / 115.  At 8192^2 (2^16) the wave kernel, bound
-// by instruction issue and the LDS there, would take four times its 4096^2
-// figures and the lane kernel 103, 140 and 221.
-constexpr int64_t DT_WAVE_MAX_BLOCKS = 1 << 14;
-// whether the phase takes less time with one wave per block than with one lane
-bool dt_wave_better(int lbx, int lby, int64_t nb, bool tinyMT);
+// Whether one wave per block is the better choice.  us per MCS (4 phases), lane /
+// wave, and the same with three simulations in flight: 512^2 (2^8 blocks) KPZ 76 /
+// 22 and 32 / 16, p/q 108 / 21 and 43 / 15, disorder 184 / 26 and 70 / 17;
+// 4096 x 2048 (2^13) 77 / 49 and 36 / 31, 110 / 48 and 53 / 33, 186 / 71 and 80 /
+// 45; 4096^2 (2^14) 78 / 82 and 37 / 57, 111 / 80 and 54 / 61, 187 / 115 and 85 /
+// 85.  From 2^14 blocks on a wave each fills the chip, bound by instruction issue
+// and the LDS, while the lanes leave three SIMDs of four to other simulations: a
+// wave each up to 2^13 blocks, and for the disorder rule up to 2^14.
+bool dt_wave_better(int lbx, int lby, int64_t nb, int upd, bool tinyMT);
 hipError_t launch_dt_wave(const DtPhaseArgs& a, const DtWaveJumps& J, hipStream_t stream);
 
 // tmtJ for a DT phase with T < nb streams: entry c < n -> x^((c / T) * drawsPerEntry)
@@ -258,10 +258,13 @@ struct BatchDtArgs {
 	const int* limit;       // optional [r]: replica r only runs MCS m < limit[r]
 };
 hipError_t launch_batch_dt(const BatchDtArgs& a, hipStream_t stream);
-// the same with one wave per block; better while all blocks that run at the
-// same time are at most DT_WAVE_MAX_BLOCKS (12 DTr jobs of L = 2^8..2^11: 67 ms
+// The same with one wave per block, better while all blocks that run at the same
+// time are at most DT_BATCH_WAVE_MAX_BLOCKS (12 DTr jobs of L = 2^8..2^11: 67 ms
 // with a lane per block, 40 so; 107 replicas of L = 2^6..2^10, 7 MCS and w^2:
-// 1.27 and 0.83 ms)
+// 1.27 and 0.83 ms; 64 replicas of L = 2^9, 2^14 blocks, 10 MCS and w^2: 1.44 and
+// 0.68).  A batch or server has its simulations in one launch, so no others are
+// reckoned with here.
+constexpr int64_t DT_BATCH_WAVE_MAX_BLOCKS = 1 << 14;
 hipError_t launch_batch_dt_wave(const BatchDtArgs& a, hipStream_t stream);
 
 struct BatchCbArgs {

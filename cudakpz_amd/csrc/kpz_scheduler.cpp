@@ -556,7 +556,7 @@ void SchedulerDT::run(int n, int upd)
 	a.random_origin = ro_;
 	a.tp = thresh(upd ? p_ : 1.0);
 	a.tq = thresh(upd ? q_ : 0.0);
-	const bool wave = dt_wave_better(lbx_, lby_, nb_, tinyMT());
+	const bool wave = dt_wave_better(lbx_, lby_, nb_, upd, tinyMT());
 	const DtWaveJumps waveJ = wave ? dt_wave_jumps(step_, du) : DtWaveJumps{};
 	for(int m = 0; m < n; ++m)
 	{

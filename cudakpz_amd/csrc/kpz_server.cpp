@@ -590,7 +590,7 @@ bool Server::enqueue(Tick& t)
 	}
 	const hipStream_t chain[2] = {s0_, s1_};
 	const bool two = nLanes_[1] > 0 || nWaves_[1] > 0;
-	const bool wave = nLanes_[0] + nLanes_[1] <= DT_WAVE_MAX_BLOCKS;
+	const bool wave = nLanes_[0] + nLanes_[1] <= DT_BATCH_WAVE_MAX_BLOCKS;
 	if(two)
 	{
 		check(hipEventRecord(fork_, s0_), "fork");

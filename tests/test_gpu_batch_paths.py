@@ -37,6 +37,19 @@ def test_batch_dt(count):
         assert np.array_equal(b.streams(i), s.streams())
 
 
+# under 2^18 blocks in all, and 2^18: draws in runs
+@pytest.mark.parametrize("count", [63, 64])
+def test_batch_dt_runs(count):
+    reps = [(K.KPZ_DT if i & 1 else K.KPZ_DTR, 11, 11, 0.6, 0.3, 50 + i) for i in range(count)]
+    b = K.Batch(reps)
+    b.initHomogeneous()
+    b.mcs(2)
+    for i in (0, 1, count - 2, count - 1):
+        s = alone(*reps[i], 2)
+        assert np.array_equal(b.popSystem(i), s.popSystem())
+        assert np.array_equal(b.streams(i), s.streams())
+
+
 # rows of 512 words: 64 lanes a row alone, 8 among many rows
 @pytest.mark.parametrize("others", [0, 40])
 def test_batch_row_split(others):

@@ -1,6 +1,6 @@
 """The kernels a double-tiling phase can take, against the oracle at the sizes
-where one hands over to the other: one wave per block (up to 2^14 blocks of
-16 x 16 sites), one lane per block above, and the lane kernel's p/q loop that
+where one hands over to the other: one wave per block (up to 2^13 or 2^14 blocks
+of 16 x 16 sites), one lane per block above, and the lane kernel's p/q loop that
 draws in runs (from 2^18 lanes on).  Everything is compared word for word."""
 import os
 
@@ -99,3 +99,16 @@ def test_draws_in_runs(ro, lx, ly):
 @pytest.mark.parametrize("ro", [False, True])
 def test_draws_in_runs_16(ro):
     run(ro, 14, 14, "pq", 1)
+
+
+# the largest lattice with a wave per block for the rules other than disorder
+@pytest.mark.parametrize("rule", ["kpz", "pq", "ew"])
+@pytest.mark.parametrize("ro", [False, True])
+def test_hand_over_of_two_draws(ro, rule):
+    run(ro, 12, 11, rule, 1)
+
+
+# 2^19 and 2^20 blocks of 4 x 4 sites: draws behind the reads, and before them
+@pytest.mark.parametrize("lx,ly", [(13, 12), (13, 13)])
+def test_draws_ahead(lx, ly):
+    run(False, lx, ly, "kpz", 2, layout=(2, 2))
