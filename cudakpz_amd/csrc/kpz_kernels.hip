@@ -628,7 +628,7 @@ __device__ __forceinline__ void dt_block(const DtPhaseArgs& a, int64_t i, int64_
 	// kpz/schedulerCPUDT_nested.h:46-66; pqOneUpdate kpz/schedulerCPU.inl:21-33)
 	// behindReads: what to do while the LDS reads are on their way
 	// LATE: the acceptance draw after the reads are issued, which for the disorder
-	// rule on a random origin is 1-2% faster with blocks below 16 x 16 (4096^2, 8 x
+	// rule on a random origin is 1-5% faster with blocks below 16 x 16 (4096^2, 8 x
 	// 8: 73.8 -> 68.5 us per MCS) and with those 3% slower (8192^2: 223 -> 231)
 	constexpr bool LATE = UPD == 2 && RO && LBX + LBY < 8;
 	auto update = [&](uint32_t d1, uint32_t d2, uint32_t d3, auto&& behindReads) {
