@@ -605,14 +605,19 @@ def main():
             steps = 100 if cls is K.SchedulerSCABit else 20
             ms = run_scabit(K, args.lx, p, q, steps, args.seed, ev, cls)
             ups = N * steps / (ms * 1e-3)
-            sec[name] = {"site_updates_per_s": ups, "hbm_GBs_algorithmic": ups * 1.0 / 1e9,
-                         "hbm_frac": ups / 1e9 / HBM_PEAK_GBS, "ms_per_mcs": ms / steps}
+            # SCABit takes a whole MCS in one pass (0.5 B per site update) in its
+            # bit-parallel mode and, from 2^31 sites on, per site; a half-sweep of
+            # its own reads and writes every word (1 B)
+            one_pass = cls is K.SchedulerSCABit and (p == 0.5 or N >= 1 << 31)
+            bpu = 0.5 if one_pass else 1.0
+            sec[name] = {"site_updates_per_s": ups, "hbm_GBs_algorithmic": ups * bpu / 1e9,
+                         "hbm_frac": ups * bpu / 1e9 / HBM_PEAK_GBS, "ms_per_mcs": ms / steps}
             if name == "scabit_p0.95_q0.05":
-                # the autocorrelator configuration's kernel: one launch per
-                # half-sweep, 2 launches per MCS, 2^31 site updates each
+                # the autocorrelator configuration's kernel: one launch per MCS,
+                # or two half-sweeps
+                kernel = "cbbit_mcs_wide_kernel<per-site>" if one_pass else "cbbit_half_kernel<u64,per-site>"
                 line["roofline_c3"] = kernel_roofline(
-                    K, f"cbbit_half_kernel<u64,per-site>@{1 << args.lx}", ms / steps / 2, 1.0 * N / 2, fast, slow,
-                    mix)
+                    K, f"{kernel}@{1 << args.lx}", ms / steps / (1 if one_pass else 2), 0.5 * N, fast, slow, mix)
         # the reference's default "dt" scheduler: DT with a random origin per
         # MCS (SchedulerCPUDTr semantics), p = 1, q = 0, 0.5 B per update
         ms = run_scabit(K, args.lx, 1.0, 0.0, 100, args.seed, ev, K.SchedulerDTr, kpz=True)
