@@ -450,8 +450,9 @@ def kernel_roofline(K, key, avg_launch_ms, algo_bytes, fast, slow, mix=None):
     run (v_xor_b32 class, kpz_valu_peak), which no instruction mix can
     exceed.  Beside it: the measured rate of the kernel's own instruction mix
     (kpz_valu_mix_rate; a fast-class instruction next to slow-class ones
-    issues at about the slow rate, so this is the bound the kernel can
-    reach), the HBM roofline (algorithmic bytes / launch time vs 8 TB/s) and
+    issues at about the slow rate, so this is the bound of a kernel whose
+    waves all have one priority; the per-site SCABit kernel draws in runs at
+    raised wave priority and passes it), the HBM roofline (algorithmic bytes / launch time vs 8 TB/s) and
     the counted HBM traffic (FETCH_SIZE + WRITE_SIZE, calibrated)."""
     prof = {}
     tfile = os.path.join(ROOT, "profiles", "traffic.json")
