@@ -796,8 +796,12 @@ void SchedulerSCABit::run(int n, int mode)
 	a.tp = thresh23(p_);
 	a.tq = thresh23(q_);
 	a.lG = lG_;
-	// (asked for on any first call: later ones may be under capture)
-	if(mode <= 1 && wholeMcs(mode))
+	// A graph keeps the addresses that it was captured with, and the spare lattice
+	// may be given back before it is replayed: half-sweeps under capture.  (Asked
+	// for on any other first call.)
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	check(hipStreamIsCapturing(stream_, &capture), "hipStreamIsCapturing");
+	if(mode <= 1 && capture == hipStreamCaptureStatusNone && wholeMcs(mode))
 	{
 		// pairs of whole MCS, so that the lattice stays where it is
 		CbMcsArgs w{};
