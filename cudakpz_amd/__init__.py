@@ -109,6 +109,19 @@ def _check(rc):
         raise KpzError(rc, lib().kpz_last_error().decode())
 
 
+def releaseSpares(device=-1):
+    """Free the second lattices that SCABit schedulers keep for MCS in one pass
+    (include/kpz_amd.h: kpz_release_spares); returns the bytes freed.  Only
+    allocations outside this library need it."""
+    L = lib()
+    L.kpz_release_spares.argtypes = [C.c_int]
+    L.kpz_release_spares.restype = C.c_int64
+    n = L.kpz_release_spares(int(device))
+    if n < 0:
+        _check(int(n))
+    return int(n)
+
+
 def _i128(lo, hi):
     return (int(hi) << 64) | (int(lo) & 0xFFFFFFFFFFFFFFFF)
 

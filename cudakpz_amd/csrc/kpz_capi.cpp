@@ -462,6 +462,17 @@ uint64_t kpz_skip(const kpz_scheduler* h) { return (h && h->s) ? h->s->skip() : 
 void* kpz_device_lattice(const kpz_scheduler* h) { return (h && h->s) ? (void*)h->s->deviceLattice() : nullptr; }
 void* kpz_stream(const kpz_scheduler* h) { return (h && h->s) ? (void*)h->s->stream() : nullptr; }
 
+int64_t kpz_release_spares(int device)
+{
+	int64_t freed = 0;
+	const int rc = guard([&] {
+		if(device < 0)
+			kpz::check(hipGetDevice(&device), "hipGetDevice");
+		freed = (int64_t)kpz::SpareBuf::takeBack(device);
+	});
+	return rc < 0 ? rc : freed;
+}
+
 int kpz_valu_peak(int device, int reps, double* slow_class, double* fast_class)
 {
 	if(!slow_class || reps < 1)

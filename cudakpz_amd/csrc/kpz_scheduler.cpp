@@ -28,10 +28,17 @@ void DevBuf::alloc(size_t bytes)
 	}
 	if(bytes == 0)
 		return;
-	const hipError_t e = hipMalloc(&p_, bytes);
+	hipError_t e = hipMalloc(&p_, bytes);
+	int device;
+	if(e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && SpareBuf::takeBack(device) > 0)
+	{
+		(void)hipGetLastError();
+		e = hipMalloc(&p_, bytes);
+	}
 	if(e != hipSuccess)
 	{
 		p_ = nullptr;
+		(void)hipGetLastError(); // the caller gets it from here, not the next launch
 		throw Error(-3, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
 	}
 	n_ = bytes;
@@ -423,17 +430,7 @@ void SchedulerService::moments(long double out[7])
 void SchedulerService::correlateTag(unsigned int stop)
 {
 	Tag t;
-	try
-	{
-		t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
-	}
-	catch(const Error&)
-	{
-		if(!dropSpare())
-			throw;
-		(void)hipGetLastError();
-		t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
-	}
+	t.snap = std::make_unique<DevBuf>(size_.sizeW() * 4);
 	t.mcs = mcs_;
 	t.stop = stop;
 	const uint64_t bytes = size_.sizeW() * 4;
@@ -658,33 +655,16 @@ SchedulerSCABit::Tables& SchedulerSCABit::tables(int mode)
 	return ref;
 }
 
-// Whether MCS of this mode run in one pass (kpz_cbbit_mcs.hip), for which the
-// scheduler keeps a second lattice.  It is taken only for lattices of at most
-// 4 GiB and only while three quarters of the device's memory stay free, so that
-// programs that fill the memory with lattices or tags find it as before.
-bool SchedulerSCABit::wholeMcs(int mode)
+// MCS in one pass (kpz_cbbit_mcs.hip) from the lattice to a spare one and back,
+// so in pairs; returns the number of MCS left to do
+int SchedulerSCABit::runWhole(int n, const CbHalfArgs& a)
 {
-	if(altState_ == NO || !cbbit_mcs_better(size_.lx, size_.ly, mode))
-		return false;
-	if(altState_ == UNKNOWN)
-	{
-		altState_ = NO;
-		const size_t bytes = (size_t)size_.sizeW() * 4;
-		size_t free = 0, total = 0;
-		if(bytes > ((size_t)4 << 30) || hipMemGetInfo(&free, &total) != hipSuccess || free < bytes ||
-		   free - bytes < total / 4 * 3)
-			return false;
-		try
-		{
-			alt_.alloc(bytes);
-		}
-		catch(const Error&)
-		{
-			(void)hipGetLastError();
-			return false;
-		}
-		altState_ = YES;
-	}
+	// a graph would keep the spare's address beyond this call
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	check(hipStreamIsCapturing(stream_, &capture), "hipStreamIsCapturing");
+	if(capture != hipStreamCaptureStatusNone)
+		return n;
+	const int mode = a.mode;
 	if(!wordJ_[mode].get())
 	{
 		std::vector<Affine> word((size_t)1 << (size_.lx - 7));
@@ -697,17 +677,37 @@ bool SchedulerSCABit::wholeMcs(int mode)
 		}
 		upload(word, wordJ_[mode]);
 	}
-	return true;
-}
-
-bool SchedulerSCABit::dropSpare()
-{
-	if(!alt_.get())
-		return false;
-	sync();
-	alt_.alloc(0);
-	altState_ = NO;
-	return true;
+	const SpareBuf::Use spare(spare_, (size_t)size_.sizeW() * 4);
+	if(!spare.get())
+		return n;
+	uint32_t* const alt = (uint32_t*)spare.get();
+	CbMcsArgs w{};
+	w.lx = size_.lx;
+	w.ly = size_.ly;
+	w.T = (int)T_;
+	w.per = per_;
+	w.rem = rem_;
+	w.rowJ = a.rowJ;
+	w.wordJ = wordJ_[mode].as<Affine>();
+	w.mode = mode;
+	w.tp = a.tp;
+	w.tq = a.tq;
+	w.step = step_;
+	w.fullBig = a.fullBig;
+	w.fullSmall = a.fullSmall;
+	w.lR = cbbit_mcs_band(size_.lx, size_.ly, mode);
+	for(; n >= 2; n -= 2)
+		for(int k = 0; k < 2; ++k)
+		{
+			w.src = k ? alt : deviceLattice();
+			w.dst = k ? deviceLattice() : alt;
+			w.st_in = stIn();
+			w.st_out = stOut();
+			check(launch_cbbit_mcs(w, stream_), "cbbit_mcs");
+			swapStreams();
+			++mcs_;
+		}
+	return n;
 }
 
 void SchedulerSCABit::run(int n, int mode)
@@ -796,41 +796,8 @@ void SchedulerSCABit::run(int n, int mode)
 	a.tp = thresh23(p_);
 	a.tq = thresh23(q_);
 	a.lG = lG_;
-	// A graph keeps the addresses that it was captured with, and the spare lattice
-	// may be given back before it is replayed: half-sweeps under capture.  (Asked
-	// for on any other first call.)
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	check(hipStreamIsCapturing(stream_, &capture), "hipStreamIsCapturing");
-	if(mode <= 1 && capture == hipStreamCaptureStatusNone && wholeMcs(mode))
-	{
-		// pairs of whole MCS, so that the lattice stays where it is
-		CbMcsArgs w{};
-		w.lx = size_.lx;
-		w.ly = size_.ly;
-		w.T = (int)T_;
-		w.per = per_;
-		w.rem = rem_;
-		w.rowJ = a.rowJ;
-		w.wordJ = wordJ_[mode].as<Affine>();
-		w.mode = mode;
-		w.tp = a.tp;
-		w.tq = a.tq;
-		w.step = step_;
-		w.fullBig = a.fullBig;
-		w.fullSmall = a.fullSmall;
-		w.lR = cbbit_mcs_band(size_.lx, size_.ly, mode);
-		for(; n >= 2; n -= 2)
-			for(int k = 0; k < 2; ++k)
-			{
-				w.src = k ? alt_.as<uint32_t>() : deviceLattice();
-				w.dst = k ? deviceLattice() : alt_.as<uint32_t>();
-				w.st_in = stIn();
-				w.st_out = stOut();
-				check(launch_cbbit_mcs(w, stream_), "cbbit_mcs");
-				swapStreams();
-				++mcs_;
-			}
-	}
+	if(cbbit_mcs_better(size_.lx, size_.ly, mode))
+		n = runWhole(n, a);
 	for(int m = 0; m < n; ++m)
 	{
 		// SchedulerCPUCBBit::doMcs (kpz/schedulerCPUCBBit.cpp:64-78)

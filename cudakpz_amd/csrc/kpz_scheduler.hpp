@@ -8,6 +8,7 @@
 #include "kpz_common.hpp"
 #include "kpz_kernels.hpp"
 #include "kpz_master.hpp"
+#include "kpz_spare.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -30,7 +31,8 @@ enum Kind { KIND_DT = 0, KIND_DTR = 1, KIND_SCABIT = 2, KIND_SCA = 3 };
 // (kpz/kpzFrontend.cpp:308-331)
 enum Rng { RNG_SLCG64 = 0, RNG_TINYMT32 = 1 };
 
-// device buffer owned by a scheduler
+// device buffer owned by a scheduler; where the memory is short it takes back
+// what the spare buffers hold (kpz_spare.hpp)
 class DevBuf {
 public:
 	DevBuf() = default;
@@ -212,8 +214,6 @@ protected:
 		std::unique_ptr<DevBuf> snap;
 		unsigned int mcs, stop;
 	};
-	// gives back memory that only makes calls faster; false if there is none
-	virtual bool dropSpare() { return false; }
 	Sums correlateWith(const DevBuf& snap);
 	void queueTotals(const uint32_t* snap, int64_t* hs); // hs: every row's start height, or null
 	Sums totals(const uint32_t* snap);
@@ -289,14 +289,12 @@ private:
 	};
 	void run(int n, int mode);
 	Tables& tables(int mode);
-	bool wholeMcs(int mode);
-	bool dropSpare() override;
+	int runWhole(int n, const CbHalfArgs& a);
 	int per_, rem_, lG_;
 	std::map<int, std::unique_ptr<Tables>> tab_;
-	// MCS in one pass: the other lattice and, per mode, the jumps to every word of
-	// a row; alt_ not asked for yet, in use, not to be had
-	DevBuf alt_, wordJ_[2];
-	enum { UNKNOWN, YES, NO } altState_ = UNKNOWN;
+	// MCS in one pass: the other lattice and, per mode, the jumps to every word of a row
+	SpareBuf spare_;
+	DevBuf wordJ_[2];
 };
 
 // Checkerboard SCA on ENC_LOCAL: SchedulerCPUCB semantics (the CPU

@@ -215,6 +215,19 @@ uint64_t kpz_skip(const kpz_scheduler* h);
 void* kpz_device_lattice(const kpz_scheduler* h);
 void* kpz_stream(const kpz_scheduler* h);
 
+/* No counterpart in the reference.  A KPZ_SCABIT scheduler runs pairs of MCS
+ * in one pass each where that is faster (kpz_mcs; kpz_mcs_pq from 2^31 sites
+ * on), for which it keeps a second lattice of the same size on the device: at
+ * most a 64th of the device's memory each and a 16th for all schedulers of a
+ * process, taken only while three quarters of the memory stay free after it,
+ * and never on a capturing stream (a graph gets half-sweeps).  Any allocation
+ * of this library that finds the memory short takes these lattices back; the
+ * results do not depend on them.  kpz_release_spares does the same for
+ * allocations that the library does not see: it frees the second lattices on
+ * `device` (-1 = current), waiting for the work queued on them, and returns
+ * the bytes freed or a negative error.  May be called from any thread. */
+int64_t kpz_release_spares(int device);
+
 /* Measurement utility, no counterpart in the reference: the integer VALU
  * issue rates of the device, the roofline that bounds the DT and per-site
  * SCA kernels, in lane operations per second (best of `reps` launches of 8

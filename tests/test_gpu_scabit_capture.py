@@ -53,6 +53,7 @@ def test_captured_mcs(lx, ly, T):
     lat = O.flat(lx, ly, O.ENC_CBBIT)
     O.cbbit_mcs(lat, lx, ly, st, 2, 0)
     for eager in (0, 2, 1, 3):
+        K.releaseSpares()
         g.replay()
         s.mcs(eager)  # the program's own steps between the replays
         s.sync()
