@@ -796,7 +796,7 @@ void SchedulerSCABit::run(int n, int mode)
 	a.tp = thresh23(p_);
 	a.tq = thresh23(q_);
 	a.lG = lG_;
-	if(cbbit_mcs_better(size_.lx, size_.ly, mode))
+	if(n >= 2 && cbbit_mcs_better(size_.lx, size_.ly, mode))
 		n = runWhole(n, a);
 	for(int m = 0; m < n; ++m)
 	{

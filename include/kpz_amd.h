@@ -217,7 +217,7 @@ void* kpz_stream(const kpz_scheduler* h);
 
 /* No counterpart in the reference.  A KPZ_SCABIT scheduler runs pairs of MCS
  * in one pass each where that is faster (kpz_mcs; kpz_mcs_pq from 2^31 sites
- * on), for which it keeps a second lattice of the same size on the device: at
+ * on), for which, from the first call of two or more MCS on, it keeps a second lattice of the same size on the device: at
  * most a 64th of the device's memory each and a 16th for all schedulers of a
  * process, taken only while three quarters of the memory stay free after it,
  * and never on a capturing stream (a graph gets half-sweeps).  Any allocation

@@ -97,6 +97,16 @@ def test_given_back_between_calls(lx, ly, T):
     assert K.releaseSpares() == 0
 
 
+def test_single_steps_take_no_spare():
+    s = seeded(15, 15, 2)
+    K.releaseSpares()
+    for _ in range(3):
+        s.mcs(1)
+    assert K.releaseSpares() == 0
+    s.mcs(3)
+    assert K.releaseSpares() >= 4 * s.size_words
+
+
 def test_given_back_by_another_thread():
     lx, ly, n = 12, 9, 600
     s = seeded(lx, ly, 6)
