@@ -664,10 +664,19 @@ int SchedulerSCABit::runWhole(int n, const CbHalfArgs& a)
 	check(hipStreamIsCapturing(stream_, &capture), "hipStreamIsCapturing");
 	if(capture != hipStreamCaptureStatusNone)
 		return n;
+	// the spare lattice, then per mode the jumps to every word of a row: one
+	// allocation, so that there is either all that the pass needs or none of it
 	const int mode = a.mode;
-	if(!wordJ_[mode].get())
+	const size_t latBytes = (size_t)size_.sizeW() * 4, words = (size_t)1 << (size_.lx - 7);
+	const SpareBuf::Use spare(spare_, latBytes + 2 * words * sizeof(Affine));
+	if(!spare.get())
+		return n;
+	if(spare.fresh())
+		wordReady_[0] = wordReady_[1] = false;
+	Affine* const wordJ = (Affine*)((char*)spare.get() + latBytes) + mode * words;
+	if(!wordReady_[mode])
 	{
-		std::vector<Affine> word((size_t)1 << (size_.lx - 7));
+		std::vector<Affine> word(words);
 		const Affine wordStep = affine_pow(step_, mode == 0 ? 2 : 64);
 		Affine acc{1, 0};
 		for(auto& j : word)
@@ -675,11 +684,10 @@ int SchedulerSCABit::runWhole(int n, const CbHalfArgs& a)
 			j = acc;
 			acc = compose(wordStep, acc);
 		}
-		upload(word, wordJ_[mode]);
+		check(hipMemcpyAsync(wordJ, word.data(), words * sizeof(Affine), hipMemcpyHostToDevice, stream_), "word jumps");
+		sync();
+		wordReady_[mode] = true;
 	}
-	const SpareBuf::Use spare(spare_, (size_t)size_.sizeW() * 4);
-	if(!spare.get())
-		return n;
 	uint32_t* const alt = (uint32_t*)spare.get();
 	CbMcsArgs w{};
 	w.lx = size_.lx;
@@ -688,7 +696,7 @@ int SchedulerSCABit::runWhole(int n, const CbHalfArgs& a)
 	w.per = per_;
 	w.rem = rem_;
 	w.rowJ = a.rowJ;
-	w.wordJ = wordJ_[mode].as<Affine>();
+	w.wordJ = wordJ;
 	w.mode = mode;
 	w.tp = a.tp;
 	w.tq = a.tq;

@@ -292,9 +292,9 @@ private:
 	int runWhole(int n, const CbHalfArgs& a);
 	int per_, rem_, lG_;
 	std::map<int, std::unique_ptr<Tables>> tab_;
-	// MCS in one pass: the other lattice and, per mode, the jumps to every word of a row
+	// MCS in one pass: the other lattice, and behind it the jump tables that are there
 	SpareBuf spare_;
-	DevBuf wordJ_[2];
+	bool wordReady_[2] = {false, false};
 };
 
 // Checkerboard SCA on ENC_LOCAL: SchedulerCPUCB semantics (the CPU

@@ -45,12 +45,13 @@ SpareBuf::~SpareBuf()
 	R.changed.notify_all();
 }
 
-void* SpareBuf::begin(size_t bytes)
+void* SpareBuf::begin(size_t bytes, bool& fresh)
 {
 	Registry& R = registry();
 	std::lock_guard<std::mutex> hold(R.lock);
 	if(recalled_ || declined_)
 		return nullptr;
+	fresh = !p_;
 	if(!p_)
 	{
 		// asked for once, and again after it was taken back

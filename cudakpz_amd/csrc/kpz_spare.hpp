@@ -25,7 +25,7 @@ public:
 	// be allocated with DevBuf: it might wait for this buffer.
 	class Use {
 	public:
-		Use(SpareBuf& b, size_t bytes) : b_(b), p_(b.begin(bytes)) {}
+		Use(SpareBuf& b, size_t bytes) : b_(b), p_(b.begin(bytes, fresh_)) {}
 		~Use()
 		{
 			if(p_)
@@ -33,10 +33,12 @@ public:
 		}
 		Use(const Use&) = delete;
 		Use& operator=(const Use&) = delete;
-		void* get() const { return p_; } // null: not to be had
+		void* get() const { return p_; }      // null: not to be had
+		bool fresh() const { return fresh_; } // nothing of an earlier use is in it
 
 	private:
 		SpareBuf& b_;
+		bool fresh_ = false;
 		void* p_;
 	};
 
@@ -44,7 +46,7 @@ public:
 	static uint64_t takeBack(int device);
 
 private:
-	void* begin(size_t bytes);
+	void* begin(size_t bytes, bool& fresh);
 	void end();
 	void* p_ = nullptr;
 	size_t n_ = 0;

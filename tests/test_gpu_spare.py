@@ -97,6 +97,20 @@ def test_given_back_between_calls(lx, ly, T):
     assert K.releaseSpares() == 0
 
 
+def test_both_rules_after_a_new_spare():
+    # 2^31 sites: both rules take one pass, each with its own table behind the spare lattice
+    s, t = seeded(17, 14, 9), seeded(17, 14, 9)
+    for k in range(3):
+        for p, q in ((0.5, 0.0), (0.9, 0.2)):
+            for x, steps in ((s, (2,)), (t, (1, 1))):
+                x.setPQ(p, q)
+                for n in steps:
+                    x.mcsPQSyncRng(n)
+        assert K.releaseSpares() >= 4 * s.size_words if k != 1 else True
+    assert sums(s) == sums(t)
+    assert np.array_equal(s.streams(), t.streams())
+
+
 def test_single_steps_take_no_spare():
     s = seeded(15, 15, 2)
     K.releaseSpares()
