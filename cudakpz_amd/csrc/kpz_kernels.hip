@@ -4012,14 +4012,28 @@ unsigned corr_grid(int64_t units)
 	const int64_t need = (units + CORR_WG / 64 - 1) / (CORR_WG / 64);
 	return (unsigned)(need < cus ? need : cus);
 }
-} // namespace
 
-// log2 of the sites from which the correlator takes the table kernel: building
-// its 129 KiB of tables takes 25 us, which the per-site kernel does not need.
-// A whole correlator sample in us, per site / tables: ENC_LOCAL 512^2 31 / 53,
-// 2048^2 35 / 56, 4096^2 (2^24) 42 / 56, 8192^2 90 / 66; ENC_CBBIT 28 / 53, 32 /
-// 51, 34 / 50, 64 / 61.
-constexpr int CORR_TABLE_MIN_LOG2 = 25;
+// Whether the correlator takes the tables of 8-site walks (row_corr_table_kernel)
+// or a wave per row and a lane per 64 sites (row_stats_kernel).  Building the
+// 129 KiB of tables takes some 25 us, which the other need not spend: always
+// tables from 2^25 sites on.  Below, a wave per row costs 2.4 ns a row however
+// narrow the row is, where the tables share a wave between rows, and walks a
+// wide row with one wave, 64 rounds at 2^18 sites.  us per correlator sample,
+// by site / by tables: ENC_LOCAL 128 x 2^13 47 / 57, x 2^14 69 / 58, x 2^17 365 /
+// 177, 2048 x 2^13 48 / 56, 32 x 2^14 49 / 56, x 2^15 75 / 70; 2^15 x 32 84 / 84,
+// 2^16 x 32 150 / 130, x 64 150 / 195, 2^18 x 64 548 / 665.  ENC_CBBIT 64 x 2^13
+// 43 / 50, x 2^14 61 / 60, x 2^18 615 / 368; 128 x 2^14 62 / 68, x 2^15 100 / 94;
+// 256 x 2^16 174 / 205; 2^14 x 32..2^11 35..48 / 43..50, 2^15 x 64 53 / 51, 2^18
+// x 64 303 / 166.
+bool corr_by_tables(int enc, int lx, int ly)
+{
+	if(lx + ly >= 25)
+		return true;
+	if(enc == ENC_LOCAL)
+		return ly > (lx < 6 ? 14 : 13) || (lx > 15 && ly < 6);
+	return lx > 14 || (lx < 8 && ly > lx + 7);
+}
+} // namespace
 
 hipError_t launch_row_stats(const uint32_t* lat, const uint32_t* snap, int enc, int lx, int ly,
 		int64_t* out, hipStream_t stream)
@@ -4027,7 +4041,7 @@ hipError_t launch_row_stats(const uint32_t* lat, const uint32_t* snap, int enc, 
 	const dim3 grid((unsigned)(((1 << ly) + 3) / 4));
 	if(enc == ENC_LOCAL)
 	{
-		if(snap && lx >= 3 && ly >= 2 && lx + ly >= CORR_TABLE_MIN_LOG2)
+		if(snap && lx >= 3 && ly >= 2 && corr_by_tables(enc, lx, ly))
 			hipLaunchKernelGGL(row_corr_table_kernel<ENC_LOCAL>, dim3(corr_grid(1ll << (ly - 2))), dim3(CORR_WG), 0,
 			                   stream, lat, snap, lx, ly, out);
 		else if(snap)
@@ -4041,7 +4055,7 @@ hipError_t launch_row_stats(const uint32_t* lat, const uint32_t* snap, int enc, 
 	}
 	else
 	{
-		if(snap && lx >= 6 && lx + ly >= CORR_TABLE_MIN_LOG2)
+		if(snap && lx >= 6 && corr_by_tables(enc, lx, ly))
 			hipLaunchKernelGGL(row_corr_table_kernel<ENC_CBBIT>, dim3(corr_grid(1ll << ly)), dim3(CORR_WG), 0,
 			                   stream,
 			                   lat, snap, lx, ly, out);

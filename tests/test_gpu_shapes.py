@@ -1,0 +1,60 @@
+"""Long and narrow lattices on the rules that choose kernels by shape: results
+against the oracle on both sides of each line, and times that may not fall off
+where a kernel is the wrong one for a shape."""
+import os
+import time
+
+import numpy as np
+import pytest
+
+import cudakpz_amd as K
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+THREADS = max(1, min(16, os.cpu_count() or 1))
+CLS = {O.ENC_LOCAL: K.SchedulerDT, O.ENC_CBBIT: K.SchedulerSCABit}
+
+
+def random_lattice(s, seed):
+    return np.random.default_rng(seed).integers(0, 1 << 32, s.size_words, dtype=np.uint64).astype(np.uint32)
+
+
+def seconds(s, f):
+    """shortest of several runs of f, waited for"""
+    best = np.inf
+    for _ in range(7):
+        s.sync()
+        t = time.perf_counter()
+        f()
+        s.sync()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("enc,lx,ly", [(O.ENC_LOCAL, 5, 14), (O.ENC_LOCAL, 5, 15), (O.ENC_LOCAL, 7, 13), (O.ENC_LOCAL, 7, 14),
+                                       (O.ENC_LOCAL, 15, 5), (O.ENC_LOCAL, 16, 5), (O.ENC_LOCAL, 16, 6),
+                                       (O.ENC_CBBIT, 6, 13), (O.ENC_CBBIT, 6, 14), (O.ENC_CBBIT, 7, 14), (O.ENC_CBBIT, 7, 15),
+                                       (O.ENC_CBBIT, 8, 16), (O.ENC_CBBIT, 14, 5), (O.ENC_CBBIT, 15, 5)])
+def test_correlate(enc, lx, ly):
+    s = CLS[enc](lx, ly)
+    snap, lat = random_lattice(s, 1), random_lattice(s, 2)
+    s.pushSystem(snap)
+    s.correlateTag()
+    s.pushSystem(lat)
+    c = s.correlate()
+    assert (c.sum_h, c.sum_hs, c.sum_h2, c.sum_hhs, c.tcs) == O.correlate_rows(lat, snap, enc, lx, ly, THREADS)
+
+
+def correlate_time(cls, lx, ly):
+    s = cls(lx, ly)
+    s.initHomogeneous()
+    s.correlateTag()
+    return seconds(s, s.correlate)
+
+
+def test_correlate_time():
+    # a quarter of the rows; with a wave for each of 2^17 narrow rows 0.64, by tables 0.31
+    assert correlate_time(K.SchedulerDT, 7, 17) < 0.5 * correlate_time(K.SchedulerDT, 7, 19)
+    # 64 rows against 128; with one wave for each long row 1.8, by tables 1.0
+    assert correlate_time(K.SchedulerSCABit, 18, 6) < 1.3 * correlate_time(K.SchedulerSCABit, 18, 7)
