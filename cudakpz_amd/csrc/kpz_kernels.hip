@@ -21,6 +21,7 @@
 
 #include "kpz_draws.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace kpz {
@@ -3054,7 +3055,7 @@ __global__ __launch_bounds__(256) void row_moments_kernel(const uint32_t* __rest
 // below 2^53, so exact) and shifts them once per round to the true heights.
 // Per 8 sites 7 table reads and 35 fp64 operations, where the per-site loop
 // took 13 fp64 and some 9 integer operations a site: a moments() call at 16384^2
-// 363 -> 156 us, at 65536^2 3.63 -> 1.60 ms (ENC_CBBIT 3.40 -> 1.20); the
+// 363 -> 143 us, at 65536^2 3.63 -> 1.51 ms (ENC_CBBIT 3.40 -> 1.20); the
 // table reads (random 8-byte LDS accesses) bound it.
 constexpr int MOMENTS = 7;
 
@@ -3167,22 +3168,28 @@ __device__ __forceinline__ void finish_moments(double (&m)[MOMENTS], double h, i
 	}
 }
 
-// one wave per word row of four site rows, taken one after the other
+// Four waves per word row, one for each of its four site rows; the workgroup
+// goes on to other word rows where there are more than MOMENT_WGS, so that its
+// table is built for several.  us per moments() call with one wave for all four
+// site rows / with a wave each: 2^18 x 64 673 / 262 (64 rows leave most of the
+// chip idle either way; by sites 499), 65536 x 256 191 / 86, 4096^2 46 / 41,
+// 16384^2 155 / 143, 65536^2 1614 / 1506; 256 x 65536 121 / 122 (124 with a
+// workgroup for each word row; with 2048 workgroups 65536^2 takes 1584).
+constexpr int MOMENT_WGS = 4096;
+
 __global__ __launch_bounds__(256) void row_moments_local_kernel(const uint32_t* __restrict__ lat, int lx, int ly,
 		const int64_t* __restrict__ hs, double* __restrict__ out)
 {
 	__shared__ double tab[MOMENTS][256];
 	build_moment_table<ENC_LOCAL>(tab);
-	__syncthreads();
-	const int yw = blockIdx.x * 4 + (threadIdx.x >> 6);
+	__syncthreads(); // the only barrier
+	const int r = threadIdx.x >> 6;
 	const int lane = threadIdx.x & 63;
-	if(yw >= (1 << (ly - 2)))
-		return; // uniform per wave; no barrier below
 	const int XW = 1 << (lx - 2);
 	const int K = XW >= 64 * 8 ? 8 : (XW > 128 ? XW / 64 : 2); // words per lane and round
-	const uint32_t* __restrict__ row = lat + ((size_t)yw << (lx - 2));
-	for(int r = 0; r < 4; ++r)
+	for(int yw = blockIdx.x; yw < (1 << (ly - 2)); yw += gridDim.x)
 	{
+		const uint32_t* __restrict__ row = lat + ((size_t)yw << (lx - 2));
 		const int64_t h0 = hs[4 * yw + r];
 		const int s0 = ((row[0] >> (8 * r)) & 1u) ? 1 : -1;
 		double sum[MOMENTS] = {0, 0, 0, 0, 0, 0, 0};
@@ -3960,8 +3967,8 @@ hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, cons
 {
 	const dim3 grid((unsigned)(((1 << ly) + 3) / 4));
 	if(enc == ENC_LOCAL && lx >= 6 && ly >= 2)
-		hipLaunchKernelGGL(row_moments_local_kernel, dim3((unsigned)(((1 << (ly - 2)) + 3) / 4)), dim3(256), 0, stream, lat,
-		                   lx, ly, hs, rows);
+		hipLaunchKernelGGL(row_moments_local_kernel, dim3((unsigned)std::min(1 << (ly - 2), MOMENT_WGS)), dim3(256), 0,
+		                   stream, lat, lx, ly, hs, rows);
 	else if(enc == ENC_CBBIT && lx >= 6)
 		hipLaunchKernelGGL(row_moments_cbbit_kernel, grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
 	else if(enc == ENC_LOCAL)

@@ -58,3 +58,28 @@ def test_correlate_time():
     assert correlate_time(K.SchedulerDT, 7, 17) < 0.5 * correlate_time(K.SchedulerDT, 7, 19)
     # 64 rows against 128; with one wave for each long row 1.8, by tables 1.0
     assert correlate_time(K.SchedulerSCABit, 18, 6) < 1.3 * correlate_time(K.SchedulerSCABit, 18, 7)
+
+
+# 2^12 word rows of four site rows, one for each workgroup, and twice to eight times as many
+@pytest.mark.parametrize("ly", [14, 15, 17])
+def test_moments_of_many_rows(ly):
+    s = K.SchedulerDT(6, ly)
+    lat = random_lattice(s, ly)
+    s.pushSystem(lat)
+    got = s.moments()
+    h = O.heights(lat, O.ENC_LOCAL, 6, ly).astype(np.int64).ravel()
+    values, counts = np.unique(h, return_counts=True)
+    for k in range(1, 8):
+        exact = sum(int(v) ** k * int(c) for v, c in zip(values, counts))
+        size = sum(abs(int(v)) ** k * int(c) for v, c in zip(values, counts))
+        # some ten roundings per site and level of the sums, each half an ulp of the absolute sum
+        assert abs(got[k - 1] * h.size - exact) <= 2.0 ** -52 * 16 * size
+
+
+def test_moments_time():
+    # 64 rows of 2^18 sites against a square of as many: 13 times as long with
+    # one wave for four of the long rows, 6 with a wave each
+    s, t = K.SchedulerDT(18, 6), K.SchedulerDT(12, 12)
+    s.initHomogeneous()
+    t.initHomogeneous()
+    assert seconds(s, s.moments) < 10 * seconds(t, t.moments)
