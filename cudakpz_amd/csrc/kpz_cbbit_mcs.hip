@@ -397,11 +397,18 @@ __global__ __launch_bounds__(MULTI ? 1024 : 256) void cbbit_mcs_wide_kernel(CbMc
 // waves.  us per MCS with targets of 1024 / 2048 / 8192 waves (8192: at least 4
 // rows): 512^2 4.6 / 4.6 / 5.9, 4096^2 5.5 / 5.5 / 6.6, 8192^2 11.4 / 9.6 / 9.6,
 // 16384^2 24.1 / 24.8 / 27.6, 32768^2 127 / 115 / 125, 65536^2 443 / 441 / 446.
+// Narrow rows have several bands in a wave, whose rows lie a band apart: with
+// 2^(lx - 7) words to a row a load takes only that part of each 128-byte line,
+// and the caches of the XCDs lose the rest before the next rows want it.  Rows of
+// up to 4 words take bands of 2 rows (256 x 2^18, 2 / 4 / 64 rows: 13.4 / 19.9 /
+// 66.3 us per MCS; 512 x 2^17 11.3 / 13.4 / 51.7), rows of 8 words up to 32
+// (1024 x 2^20, 32 / 64 rows: 172 / 214; x 2^22 679 / 665).
 int cbbit_mcs_band(int lx, int ly, int mode)
 {
 	if(mode == 1)
 		return ly < 5 ? ly : 5; // 65536^2: 962 us per MCS with 16 rows, 912 with 32, 923 with 64
-	int lR = ly < 6 ? ly : 6;
+	const int most = lx < 10 ? 1 : (lx == 10 ? 5 : 6);
+	int lR = ly < most ? ly : most;
 	const int lanes = lx <= 13 ? lx - 7 : lx - 8; // log2 lanes per band
 	while(lR > 1 && ((1ll << (ly - lR + lanes)) >> 6) < 2048)
 		--lR;

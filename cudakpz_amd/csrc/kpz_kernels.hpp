@@ -107,9 +107,16 @@ int cbbit_mcs_band(int lx, int ly, int mode); // log2 rows of a band
 // pass pays from 2^31 sites on, where its bands of 32 rows fill the chip.  us per
 // MCS in half-sweeps / one pass, p = .95 q = .05 and q = 0: 65536^2 1021 / 912,
 // 890 / 761; 65536 x 32768 542 / 505, 471 / 414; 32768^2 294 / 301, 237 / 254.
+// The bit-parallel one pays on all rows of 8 words and more (1024 x 2^20, 1000
+// workers, 185 / 162); on narrower ones, whose bands have to be short and read
+// twice what they write, while lattice and spare stay in the caches of the XCDs:
+// 256 x 2^18 (2^26 sites) 15 / 13, 512 x 2^17 16 / 11, but 256 x 2^19, 1000
+// workers, 22 / 24, 128 x 2^22 107 / 114, 256 x 2^21 96 / 101.
 inline bool cbbit_mcs_better(int lx, int ly, int mode)
 {
-	return lx >= 7 && lx <= CBBIT_MCS_MAX_LX && (mode == 0 || (mode == 1 && lx >= 15 && lx + ly >= 31));
+	if(lx < 7 || lx > CBBIT_MCS_MAX_LX)
+		return false;
+	return mode == 0 ? lx >= 10 || lx + ly <= 26 : mode == 1 && lx >= 15 && lx + ly >= 31;
 }
 struct CbMcsArgs {
 	const uint32_t* src;

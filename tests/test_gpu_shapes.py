@@ -83,3 +83,30 @@ def test_moments_time():
     s.initHomogeneous()
     t.initHomogeneous()
     assert seconds(s, s.moments) < 10 * seconds(t, t.moments)
+
+
+# rows of 1 to 8 words on tall lattices: one pass in bands of 2 rows up to 2^26
+# sites, half-sweeps above; rows of 8 words in one pass throughout
+@pytest.mark.parametrize("lx,ly,T", [(7, 19, 0), (8, 18, 1000), (9, 17, 0), (9, 18, 7), (10, 17, 1000)])
+def test_tall_scabit(lx, ly, T):
+    s = K.SchedulerSCABit(lx, ly, threads=T)
+    s.supplySeed(12)
+    s.initHomogeneous()
+    s.mcs(2)
+    s.mcs(3)
+    m = O.Dsfmt(O.seed32(12))
+    st = O.Streams(s.threads, m)
+    lat = O.flat(lx, ly, O.ENC_CBBIT)
+    O.cbbit_mcs_threaded(lat, lx, ly, st, 5, 0, 0.5, 0.0, THREADS)
+    assert np.array_equal(s.popSystem(), lat)
+    assert np.array_equal(s.streams(), st.states)
+
+
+@pytest.mark.parametrize("lx,ly", [(7, 22), (8, 18), (8, 20), (9, 18), (10, 20)])
+def test_tall_scabit_time(lx, ly):
+    # ten MCS in one call against ten calls of one, which are half-sweeps
+    # (3 to 6 times as long on rows of 1 and 2 words with bands of 16 and more rows)
+    s = K.SchedulerSCABit(lx, ly)
+    s.initHomogeneous()
+    s.mcs(2)
+    assert seconds(s, lambda: s.mcs(10)) < 1.2 * seconds(s, lambda: [s.mcs(1) for _ in range(10)])
