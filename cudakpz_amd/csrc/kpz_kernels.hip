@@ -3969,12 +3969,12 @@ hipError_t launch_row_moments(const uint32_t* lat, int enc, int lx, int ly, cons
 	if(enc == ENC_LOCAL && lx >= 6 && ly >= 2)
 		hipLaunchKernelGGL(row_moments_local_kernel, dim3((unsigned)std::min(1 << (ly - 2), MOMENT_WGS)), dim3(256), 0,
 		                   stream, lat, lx, ly, hs, rows);
-	else if(enc == ENC_CBBIT && lx >= 6)
-		hipLaunchKernelGGL(row_moments_cbbit_kernel, grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
 	else if(enc == ENC_LOCAL)
 		hipLaunchKernelGGL((row_moments_kernel<ENC_LOCAL>), grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
+	else if(lx >= 6)
+		hipLaunchKernelGGL(row_moments_cbbit_kernel, grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
 	else
-		hipLaunchKernelGGL((row_moments_kernel<ENC_CBBIT>), grid, dim3(256), 0, stream, lat, lx, ly, hs, rows);
+		return hipErrorInvalidValue; // no such lattice
 	hipLaunchKernelGGL(moments_group_kernel, dim3((unsigned)moment_groups(ly)), dim3(64), 0, stream, rows, 1 << ly, groups);
 	return hipGetLastError();
 }
