@@ -136,7 +136,8 @@ def run_reductions(K, lx, seed, reps=5):
 
 
 def run_scabit(K, lx, p, q, steps, seed, ev, cls=None, kpz=False, rng=0, threads=0):
-    """steps MCS of mcsPQSyncRng (kpz: mcs) after 2 warm-up MCS, hipEvent time.
+    """steps MCS of mcsPQSyncRng (kpz: mcs) after 2 warm-up MCS: hipEvent time in
+    ms, and whether they ran in one pass each (SCABit).
     rng = TinyMT32: the engine's default worker count, parameter set t of
     stream t = random words (the reference's table is not in its tree)"""
     s = (cls or K.SchedulerSCABit)(lx, lx, rng=rng, threads=threads)
@@ -153,9 +154,9 @@ def run_scabit(K, lx, p, q, steps, seed, ev, cls=None, kpz=False, rng=0, threads
     ev.record(a, s.stream)
     run(steps)
     ev.record(b, s.stream)
-    ms = ev.ms(a, b)
+    ms, one_pass = ev.ms(a, b), s.onePass()
     s.close()
-    return ms
+    return ms, one_pass
 
 
 def batch_mix(n=4096, base_seed=1000, umin=6, umax=11, rng_seed=4096):
@@ -604,12 +605,10 @@ def main():
                                 ("scabit_p0.95_q0.05", 0.95, 0.05, K.SchedulerSCABit),
                                 ("sca_local_p0.95_q0", 0.95, 0.0, K.SchedulerSCA)]:
             steps = 100 if cls is K.SchedulerSCABit else 20
-            ms = run_scabit(K, args.lx, p, q, steps, args.seed, ev, cls)
+            ms, one_pass = run_scabit(K, args.lx, p, q, steps, args.seed, ev, cls)
             ups = N * steps / (ms * 1e-3)
-            # SCABit takes a whole MCS in one pass (0.5 B per site update) in its
-            # bit-parallel mode and, from 2^31 sites on, per site; a half-sweep of
+            # a whole MCS in one pass moves 0.5 B per site update, a half-sweep of
             # its own reads and writes every word (1 B)
-            one_pass = cls is K.SchedulerSCABit and (p == 0.5 or N >= 1 << 31)
             bpu = 0.5 if one_pass else 1.0
             sec[name] = {"site_updates_per_s": ups, "hbm_GBs_algorithmic": ups * bpu / 1e9,
                          "hbm_frac": ups * bpu / 1e9 / HBM_PEAK_GBS, "ms_per_mcs": ms / steps}
@@ -621,7 +620,7 @@ def main():
                     K, f"{kernel}@{1 << args.lx}", ms / steps / (1 if one_pass else 2), 0.5 * N, fast, slow, mix)
         # the reference's default "dt" scheduler: DT with a random origin per
         # MCS (SchedulerCPUDTr semantics), p = 1, q = 0, 0.5 B per update
-        ms = run_scabit(K, args.lx, 1.0, 0.0, 100, args.seed, ev, K.SchedulerDTr, kpz=True)
+        ms, _ = run_scabit(K, args.lx, 1.0, 0.0, 100, args.seed, ev, K.SchedulerDTr, kpz=True)
         ups = N * 100 / (ms * 1e-3)
         sec["dtr_p1_q0"] = {"site_updates_per_s": ups, "hbm_GBs_algorithmic": ups * 0.5 / 1e9,
                             "hbm_frac": ups * 0.5 / 1e9 / HBM_PEAK_GBS, "ms_per_mcs": ms / 100}
@@ -638,7 +637,7 @@ def main():
                 ("dtr_tinymt32_T32_p1_q0", K.SchedulerDTr, True, 1.0, 0.0, 20, 0.5, 32),
                 ("scabit_tinymt32_T32_p0.5_q0", K.SchedulerSCABit, True, 0.5, 0.0, 20, 1.0, 32),
                 ("sca_tinymt32_T32_p0.95_q0", K.SchedulerSCA, True, 0.95, 0.0, 10, 1.0, 32)):
-            ms = run_scabit(K, args.lx, p, q, steps, args.seed, ev, cls, kpz=kpz, rng=K.RNG_TINYMT32, threads=T)
+            ms, _ = run_scabit(K, args.lx, p, q, steps, args.seed, ev, cls, kpz=kpz, rng=K.RNG_TINYMT32, threads=T)
             ups = N * steps / (ms * 1e-3)
             sec[name] = {"site_updates_per_s": ups, "hbm_GBs_algorithmic": ups * bpu / 1e9,
                          "hbm_frac": ups * bpu / 1e9 / HBM_PEAK_GBS, "ms_per_mcs": ms / steps}

@@ -313,6 +313,16 @@ class SchedulerService:
     def mcsPQ(self, n):
         self.mcsPQSyncRng(n)
 
+    def onePass(self):
+        """Whether the last mcs / mcsPQSyncRng call ran in one pass per MCS
+        (SCABit; include/kpz_amd.h: kpz_one_pass)."""
+        L = lib()
+        L.kpz_one_pass.argtypes = [C.c_void_p]
+        rc = L.kpz_one_pass(self._h)
+        if rc < 0:
+            _check(rc)
+        return bool(rc)
+
     def mcsScale(self):
         return float(lib().kpz_mcs_scale(self._h))
 

@@ -462,6 +462,12 @@ uint64_t kpz_skip(const kpz_scheduler* h) { return (h && h->s) ? h->s->skip() : 
 void* kpz_device_lattice(const kpz_scheduler* h) { return (h && h->s) ? (void*)h->s->deviceLattice() : nullptr; }
 void* kpz_stream(const kpz_scheduler* h) { return (h && h->s) ? (void*)h->s->stream() : nullptr; }
 
+int kpz_one_pass(const kpz_scheduler* h)
+{
+	HANDLE(h);
+	return h->s->onePass() ? 1 : 0;
+}
+
 int64_t kpz_release_spares(int device)
 {
 	int64_t freed = 0;

@@ -704,6 +704,7 @@ int SchedulerSCABit::runWhole(int n, const CbHalfArgs& a)
 	w.fullBig = a.fullBig;
 	w.fullSmall = a.fullSmall;
 	w.lR = cbbit_mcs_band(size_.lx, size_.ly, mode);
+	onePass_ = true;
 	for(; n >= 2; n -= 2)
 		for(int k = 0; k < 2; ++k)
 		{
@@ -722,6 +723,7 @@ void SchedulerSCABit::run(int n, int mode)
 {
 	if(mode == 2 && !hasDisorder())
 		throw Error(-4, "mcsDisorder2SyncRng needs a disorder map (generateDisorder2 / setDisorder)");
+	onePass_ = false;
 	if(tinyMT())
 	{
 		// TinyMT32 workers: per half-sweep the random part first (one lane per

@@ -127,6 +127,7 @@ public:
 	virtual void mcsPQSyncRng(int n) = 0;    // general p, q
 	void mcsPQ(int n) { mcsPQSyncRng(n); }
 	virtual double mcsScale() const { return 1.0; }
+	virtual bool onePass() const { return false; } // the last call's MCS took one pass each (SCABit)
 	unsigned int mcsCount() const { return mcs_; }
 	void setMcs(unsigned int m) { mcs_ = m; }
 
@@ -281,6 +282,7 @@ public:
 	void mcsPQSyncRng(int n) override;       // bit-parallel if (.5, 0), else per site
 	void mcsDisorder2SyncRng(int n) override;
 	double mcsScale() const override { return p_ + q_; }
+	bool onePass() const override { return onePass_; }
 
 private:
 	struct Tables {
@@ -295,6 +297,7 @@ private:
 	// MCS in one pass: the other lattice, and behind it the jump tables that are there
 	SpareBuf spare_;
 	bool wordReady_[2] = {false, false};
+	bool onePass_ = false;
 };
 
 // Checkerboard SCA on ENC_LOCAL: SchedulerCPUCB semantics (the CPU

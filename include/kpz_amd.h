@@ -227,6 +227,10 @@ void* kpz_stream(const kpz_scheduler* h);
  * `device` (-1 = current), waiting for the work queued on them, and returns
  * the bytes freed or a negative error.  May be called from any thread. */
 int64_t kpz_release_spares(int device);
+/* 1 if the last kpz_mcs / kpz_mcs_pq call ran its MCS (but an odd last one) in
+ * one pass each, 0 if in half-sweeps or by another scheduler; for accounts of
+ * the memory moved */
+int kpz_one_pass(const kpz_scheduler* h);
 
 /* Measurement utility, no counterpart in the reference: the integer VALU
  * issue rates of the device, the roofline that bounds the DT and per-site

@@ -143,3 +143,27 @@ def test_given_back_by_another_thread():
     O.cbbit_mcs_threaded(lat, lx, ly, st, n, 0, 0.5, 0.0, 8)
     assert np.array_equal(s.popSystem(), lat)
     assert np.array_equal(s.streams(), st.states)
+
+
+# what bench.py accounts the memory by: the width and size limits of the rule,
+# a row wider than the one-pass kernel takes, a spare that is not to be had
+@pytest.mark.parametrize("lx,ly,rule,one", [(6, 9, "mcs", False), (7, 9, "mcs", True), (18, 5, "mcs", True), (19, 5, "mcs", False),
+                                            (12, 12, "pq", False), (14, 17, "pq", False), (15, 16, "pq", True)])
+def test_one_pass_is_told(lx, ly, rule, one):
+    s = seeded(lx, ly, 1)
+    s.setPQ(0.9, 0.1)
+    advance = s.mcs if rule == "mcs" else s.mcsPQSyncRng
+    advance(2)
+    assert s.onePass() is one
+    advance(1)
+    assert s.onePass() is False
+    assert K.SchedulerDT(8, 8).onePass() is False
+
+
+def test_no_spare_is_told():
+    s = seeded(18, 16, 1)  # 4 GiB: as large as a spare may be
+    s.mcs(2)
+    assert s.onePass()
+    t = seeded(18, 17, 1)  # 8 GiB
+    t.mcs(2)
+    assert not t.onePass()
