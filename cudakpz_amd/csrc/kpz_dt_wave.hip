@@ -16,11 +16,11 @@
 // after all earlier ones that it depends on, so applying level after level,
 // window after window gives the sequential result bit for bit.  An update
 // that accepts neither a minimum nor a maximum changes nothing and is left
-// out.  Random sites need 5-6 levels per window, 20-24 per block, against 256
-// sequential steps.
+// out.  Random sites need 4.3 levels per window, 17 (12 to 25) per block, against
+// 256 sequential steps.
 //
 // What bounds it: latency (the lattice and stream loads, the LDS round trips
-// of the level search, 20-24 dependent steps of 9 instructions) on small
+// of the level search, some 17 dependent steps of 9 instructions) on small
 // lattices; from 4096^2 on VALU issue (about 700 instructions per block) and the
 // LDS (random 8-byte accesses, 28 per block and lane).  Tried and not kept: four
 // blocks per wave, levelled one after the other and applied together by 16

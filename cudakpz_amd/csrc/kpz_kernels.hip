@@ -3392,7 +3392,10 @@ __global__ __launch_bounds__(256) void copy_kernel(uint4* __restrict__ dst, cons
 // RO: the DTr lanes [nstatic, nlanes), else the static DT lanes [0, nstatic):
 // one kernel per kind, so that the static DT lanes keep the register budget
 // (and occupancy) of the static update loop rather than the DTr staging's
-// PQ: the loop of the p/q rule (DT_RUNS_MIN_LANES)
+// PQ: the loop of the p/q rule (DT_RUNS_MIN_LANES).  The KPZ rule draws before
+// the update whatever the launch: mixed batches of 128 to 4096 replicas take the
+// same time with the draws behind the reads (1024: 4.60 / 4.60 ms for 10 MCS),
+// batches of KPZ alone up to 17 % less (20 of 2048^2 1.26 / 1.05, 256 6.25 / 6.28).
 template<bool RO, DtLoop PQ>
 __global__ __launch_bounds__(DT_WG) void batch_dt_kernel(BatchDtArgs a)
 {
@@ -3697,7 +3700,7 @@ __global__ __launch_bounds__(BC_WG) void batch_combine_kernel(const BatchRep* __
 // per MCS, p = q = .5, without and with, static and random origin: 8192^2 (2^16
 // lanes, a wave per SIMD) 0.139 / 0.149 and 0.156 / 0.174; 16384^2 (2^18) 0.310
 // / 0.266 and 0.304 / 0.265; 65536^2 4.08 / 3.65 and 3.74 / 3.48; a batch of
-// 1024 replicas, half of its DT blocks p/q, 6.00 / 5.83.  The disorder rule
+// 1024 replicas, half of its DT blocks p/q, the same within its runs' spread.  The disorder rule
 // loses with the runs (16384^2 0.52 / 0.56), and the rules of two draws gain
 // nothing (65536^2 2.65 / 2.67): their LDS accesses, 7.7 ns per wave and update,
 // bound the chip to 2.1 T updates/s.

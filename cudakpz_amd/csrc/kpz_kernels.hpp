@@ -56,8 +56,11 @@ DtWaveJumps dt_wave_jumps(const Affine& step, int drawsPerUpdate);
 // 4096 x 2048 (2^13) 77 / 49 and 36 / 31, 110 / 48 and 53 / 33, 186 / 71 and 80 /
 // 45; 4096^2 (2^14) 78 / 82 and 37 / 57, 111 / 80 and 54 / 61, 187 / 115 and 85 /
 // 85.  From 2^14 blocks on a wave each fills the chip, bound by instruction issue
-// and the LDS, while the lanes leave three SIMDs of four to other simulations: a
-// wave each up to 2^13 blocks, and for the disorder rule up to 2^14.
+// and the LDS, while the lanes leave three SIMDs of four to other simulations.
+// There KPZ takes half as long again with a wave each while others are in flight
+// (random origin 86 / 79 and 39 / 58); p/q gains 28 % alone and loses 13 % with
+// others, where 61 is more than the lane kernel ever took (58): a wave each up to
+// 2^13 blocks, and for the disorder rule up to 2^14.
 bool dt_wave_better(int lbx, int lby, int64_t nb, int upd, bool tinyMT);
 hipError_t launch_dt_wave(const DtPhaseArgs& a, const DtWaveJumps& J, hipStream_t stream);
 

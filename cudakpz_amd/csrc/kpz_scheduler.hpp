@@ -141,7 +141,8 @@ public:
 	// ---- measurements (exact, on device)
 	Sums roughness();
 	// height moments <h^k>, k = 1..7, as Roughness::h[] after normAndSetW2
-	// (kpz/roughness.cpp:38-43): per-row double sums, rows added in long double
+	// (kpz/roughness.cpp:38-43): per-row double sums, 64 rows at a time added with
+	// their rounding errors on the device, and those in long double
 	void moments(long double out[7]);
 	// correlateTag(stop) (kpz/schedulerService.cpp:266-271): a device snapshot
 	// kept while mcs <= stop; several tags may be live at once

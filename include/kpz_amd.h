@@ -150,8 +150,9 @@ int kpz_roughness(kpz_scheduler* h, int64_t out[3]);
  * or events). */
 int kpz_roughness_noalloc(const uint32_t* lattice, int lx, int ly, int encoding, int64_t* out, void* stream);
 /* height moments <h^k>, k = 1..7 (Roughness::h[] after normAndSetW2,
- * kpz/roughness.cpp:38-43, kpz/schedulerService.h:52-71): per-row double
- * sums on the device, rows added in long double; the 7 values the
+ * kpz/roughness.cpp:38-43, kpz/schedulerService.h:52-71): sums in
+ * double, 64 rows at a time added up on the device as value and rounding
+ * error, those in long double; the 7 values the
  * reference prints after w^2 (operator<< of Roughness,
  * kpz/schedulerService.cpp:73-79) */
 int kpz_moments(kpz_scheduler* h, double out[7]);
@@ -245,8 +246,9 @@ int kpz_valu_peak(int device, int reps, double* slow_class, double* fast_class);
  * VALU instructions of which slow_of_8 (0, 2, 3, 4, 5 or 8) are v_mul_lo_u32
  * (slow class) and the rest v_xor_b32 (fast class), 8 waves per SIMD.  On
  * gfx950 a fast-class instruction next to slow-class ones issues at about the
- * slow rate, so this, at a kernel's own slow fraction, is the VALU roofline
- * of that kernel. */
+ * slow rate, so this, at a kernel's own slow fraction, bounds a kernel whose
+ * waves all have one priority; one that gathers its slow-class instructions in
+ * runs at raised wave priority (the per-site SCABit rule) passes it. */
 int kpz_valu_mix_rate(int device, int reps, int slow_of_8, double* lane_ops_per_s);
 
 /* ---------------------------------------------------------------------
@@ -276,7 +278,8 @@ typedef struct kpz_batch_tuning {
 	int sort_by_size;   /* large replicas first */
 } kpz_batch_tuning;
 
-/* tuning = NULL: defaults {3, 1, 50, 2, 1} */
+/* tuning = NULL: {L, 1, 50, 2, 1} with L chosen for the batch: 3, and up to 6
+ * where 8 lanes per row would leave the SCABit rows fewer than 4096 waves */
 int kpz_batch_create(const kpz_replica* reps, int n, const kpz_batch_tuning* tuning, int device, kpz_batch** out);
 int kpz_batch_destroy(kpz_batch* b);
 int kpz_batch_init_flat(kpz_batch* b);
